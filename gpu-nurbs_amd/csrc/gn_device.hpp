@@ -4,6 +4,31 @@
 
 namespace gn {
 
+// A pointer read from memory (an object or request table) is generic to the compiler, whose accesses
+// through it then are flat ones: they check the LDS aperture and are waited for together with LDS
+// accesses.  These tables hold pointers to device memory only: global_view reads a table's entry
+// with its pointers as such.  `slot` is the pointer's place in the table.
+template <typename P>
+__device__ __forceinline__ P *load_global(P *const &slot) {
+    __attribute__((address_space(1))) P *g;
+    __builtin_memcpy(&g, &slot, sizeof(g));
+    return (P *)g;
+}
+__device__ __forceinline__ GnCurveDev global_view(const GnCurveDev &s) {
+    GnCurveDev c = s;
+    c.k = load_global(s.k);
+    c.ih = load_global(s.ih);
+    c.tab64 = load_global(s.tab64);
+    c.tab32 = load_global(s.tab32);
+    c.samp = load_global(s.samp);
+    c.samp_t = load_global(s.samp_t);
+    return c;
+}
+__device__ __forceinline__ GnReq global_view(const GnReq &s) {
+    return GnReq{load_global(s.x), load_global(s.y), load_global(s.z), load_global(s.u),
+                 load_global(s.v), load_global(s.status), load_global(s.it32), load_global(s.it64)};
+}
+
 // Knot-span lookup.  Returns the unique m with k[m] <= u < k[m+1], clamped to [p, cp-1] exactly
 // as findSpan (src/NURBS/Evaluate.cu:504-533): u >= k[cp] -> cp-1, u <= k[p] -> p.  A NaN makes
 // the reference's while-loop exit at its first midpoint, (p + cp) / 2; that is reproduced too.

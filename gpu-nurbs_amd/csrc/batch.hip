@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kSeedBlock) void k_batch_seed(const GnBatchObj *__r
     __shared__ __align__(16) float lbox[(((1 << (2 * (kBatchSeedLdsLevels + 1))) - 1) / 3 - 1) * 6];
     for (long long b = blockIdx.x; b < nblocks; b += gridDim.x) {  // workgroup-uniform
         const GnTile tl = tiles[b / per_tile];
-        const GnSearchDev &sd = objs[tl.obj].sd;
+        const GnSearchDev sd = global_view(objs[tl.obj].sd);
         const int ll = mode == GN_SEED_NEAREST_LEAF || mode == GN_SEED_GRID_STEP
                            ? 0
                            : (sd.depth < kBatchSeedLdsLevels ? sd.depth : kBatchSeedLdsLevels);
@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kSeedBlock) void k_batch_seed(const GnBatchObj *__r
         __syncthreads();
         const int j = (int)(b % per_tile) * kSeedBlock + threadIdx.x;
         if (j >= tl.count) continue;
-        const GnReq &R = reqs[tl.req];
+        const GnReq R = global_view(reqs[tl.req]);
         const int64_t i = tl.start + j;
         const double P[3] = {R.x[i], R.y[i], R.z[i]};
         if (mode == GN_SEED_GRID_STEP) {  // the object (and its grid's width) is workgroup-uniform
@@ -199,8 +199,8 @@ void k_batch(BatchArgs a, unsigned long long *counters, int slices, int max_iter
                 if (rank < avail) {
                     idx = q_lo + (long long)rank;
                     rq = cur_req;
-                    d = a.objs[cur_obj].s;
-                    const GnReq &R = a.reqs[cur_req];
+                    d = global_view(a.objs[cur_obj].s);
+                    const GnReq R = global_view(a.reqs[cur_req]);
                     Px = T(R.x[idx]);
                     Py = T(R.y[idx]);
                     Pz = T(R.z[idx]);
@@ -226,7 +226,7 @@ void k_batch(BatchArgs a, unsigned long long *counters, int slices, int max_iter
         if (WAVE && cur_cls < 16) {
             // the whole wave steps (cur_cls is wave-uniform); a lane with no step due evaluates
             // the wave's current surface at its domain corner and discards the result
-            const GnSurfDev dd = act ? d : a.objs[cur_obj].s;
+            const GnSurfDev dd = act ? d : global_view(a.objs[cur_obj].s);
             double tu = act ? cu : dd.ku[dd.p], tv = act ? cv : dd.kv[dd.q];
             const int s2 = step_group<GRP, T, NEWTON, PREG, true>(
                 cur_cls, dd, act ? Px : T(0), act ? Py : T(0), act ? Pz : T(0), tu, tv, tol_dist,
@@ -252,7 +252,7 @@ void k_batch(BatchArgs a, unsigned long long *counters, int slices, int max_iter
                     cu = su;
                     cv = sv;
                 }
-                const GnReq &R = a.reqs[rq];
+                const GnReq R = global_view(a.reqs[rq]);
                 R.u[idx] = cu;
                 R.v[idx] = cv;
                 R.status[idx] = (uint8_t)st;

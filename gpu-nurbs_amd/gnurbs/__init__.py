@@ -303,7 +303,7 @@ class Surface:
         return out, perm
 
     def EvaluateGrid(self, us, vs, order: int = 0, out=None, stream=None):
-        """FP32 MFMA span-GEMM evaluation on the grid us x vs; returns (nblk, len(us)*len(vs))."""
+        """FP32 evaluation on the grid us x vs; returns (nblk, len(us)*len(vs))."""
         torch = _torch()
         ud, vd = to_device(us, torch.float32), to_device(vs, torch.float32)
         nblk = (3, 9, 18)[order] if 0 <= order <= 2 else 3

@@ -163,7 +163,7 @@ int gn_evaluate(const gn_surface *s, const double *u, const double *v, size_t n,
 /* FP32 form: parameters are floats (span lookup still compares against FP64 knots). */
 int gn_evaluate_f32(const gn_surface *s, const float *u, const float *v, size_t n,
                     int max_order, float *out, gn_stream stream);
-/* Tensor-product grid (us[nu_pts] x vs[nv_pts]), FP32 MFMA span-GEMM form; out SoA blocks of
+/* Tensor-product grid (us[nu_pts] x vs[nv_pts]), FP32 span-GEMM form; out SoA blocks of
  * nu_pts*nv_pts values, point (a, b) at a*nv_pts + b.  us, vs ascending; max_order 0..2. */
 int gn_evaluate_grid_f32(const gn_surface *s, const float *us, int nu_pts, const float *vs,
                          int nv_pts, int max_order, float *out, gn_stream stream);

@@ -48,7 +48,8 @@ struct GnSearchDev {
     const float4 *rec;        // per leaf (Morton order) one 128-byte record (kRecVec vectors) for
                               // the stepped seeds, one cache line: [0] as leaf32, [1] the seed
                               // (u, v) as two doubles, [2..6] S_u, S_v, S_uu, S_uv, S_vv at the
-                              // seed in FP32 (w = 0), [7] zero
+                              // seed in FP32 (w = 0), [7] cos^2 of the normal cone's widened
+                              // half-angle (double), then zero
     const float4 *cone32;     // per leaf (Morton order) normal cone: unit axis, half-angle
                               // (radians, rounded up; 4 when unbounded); null: no cone pruning
     double u0, u1, v0, v1;    // the knot domain the leaves tile

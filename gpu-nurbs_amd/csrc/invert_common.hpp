@@ -125,17 +125,11 @@ __device__ __forceinline__ Domain domain_of(const GnSurfDev &d) {
 // direction points outward is held and the other takes its one-dimensional step, with the exact
 // one-dimensional second derivative where that is positive (a plain clamp of the coupled step can
 // walk uphill along an edge).  rr_out: the squared residual at the point evaluated.
-template <int K1, int K2, bool EXACT, typename T, bool NEWTON, int PSRC = kPatchGlobal,
-          bool ACTIVE = false, bool NEAR = false>
-__device__ __forceinline__ int gn_step(const GnSurfDev &d, const double *__restrict__ ku,
-                                       const double *__restrict__ kv, T Px, T Py, T Pz,
-                                       double &cu, double &cv, double tol_dist, double tol_step,
-                                       double tol_quad, int clamp, const Domain &dom,
-                                       SpanCache &sc, Hom<T> *pr = nullptr,
-                                       float4 *wave_lds = nullptr, T *rr_out = nullptr) {
-    Cart<T> o;
-    eval_point_cached<K1, K2, NEWTON ? 2 : 1, EXACT, T, PSRC, NEAR>(d, ku, kv, cu, cv, sc, o, pr,
-                                                              wave_lds);
+template <typename T, bool NEWTON, bool ACTIVE = false>
+__device__ __forceinline__ int gn_update(const GnSurfDev &d, const Cart<T> &o, T Px, T Py, T Pz,
+                                         double &cu, double &cv, double tol_dist, double tol_step,
+                                         double tol_quad, int clamp, const Domain &dom,
+                                         const SpanCache &sc, T *rr_out = nullptr) {
     const T r0 = o.S[0] - Px, r1 = o.S[1] - Py, r2 = o.S[2] - Pz;
     const T rr = r0 * r0 + r1 * r1 + r2 * r2;
     if (rr_out) *rr_out = rr;
@@ -215,6 +209,22 @@ __device__ __forceinline__ int gn_step(const GnSurfDev &d, const double *__restr
             return GN_PT_CONVERGED;
     }
     return kStepContinue;
+}
+
+// The surface at (cu, cv), then the update.
+template <int K1, int K2, bool EXACT, typename T, bool NEWTON, int PSRC = kPatchGlobal,
+          bool ACTIVE = false, bool NEAR = false>
+__device__ __forceinline__ int gn_step(const GnSurfDev &d, const double *__restrict__ ku,
+                                       const double *__restrict__ kv, T Px, T Py, T Pz,
+                                       double &cu, double &cv, double tol_dist, double tol_step,
+                                       double tol_quad, int clamp, const Domain &dom,
+                                       SpanCache &sc, Hom<T> *pr = nullptr,
+                                       float4 *wave_lds = nullptr, T *rr_out = nullptr) {
+    Cart<T> o;
+    eval_point_cached<K1, K2, NEWTON ? 2 : 1, EXACT, T, PSRC, NEAR>(d, ku, kv, cu, cv, sc, o, pr,
+                                                              wave_lds);
+    return gn_update<T, NEWTON, ACTIVE>(d, o, Px, Py, Pz, cu, cv, tol_dist, tol_step, tol_quad,
+                                        clamp, dom, sc, rr_out);
 }
 
 // Up to max_iter steps from (cu, cv); *iters = updates performed.

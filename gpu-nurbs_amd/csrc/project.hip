@@ -8,7 +8,7 @@
 //   2. every leaf whose FP32 box (a conservative lower bound) is not farther than the best foot
 //      point so far, and whose normal cone allows a foot point inside it (cone_may_hold; leaves
 //      on the domain boundary, where the nearest point need not be a foot point, always pass),
-//      gets a projected Newton solve clamped to its uv cell, from the cell centre; a nearer
+//      gets a projected Newton solve clamped to its uv cell, from the leaf's stepped seed; a nearer
 //      result tightens the bound, which prunes the rest of the depth-first walk;
 //   3. the nearest foot point is polished by projected Newton over the whole domain (kept unless it
 //      is farther by more than rounding, 1e-9 relative in squared distance).
@@ -16,7 +16,7 @@
 // depth-3 tree (64 x 64 cells) are nearly flat, so the distance restricted to one is close to
 // convex.  Projected Newton (gn_step with ACTIVE) holds a coordinate on its bound while the
 // descent points outward, so minima on cell edges and on the surface boundary are reached too.
-// FP64, one lane per query, exact-Hessian steps.  Also the fallback of gn_invert (opts.fallback):
+// FP64, exact-Hessian steps.  Also the fallback of gn_invert (opts.fallback):
 // the queries an inversion left unconverged are listed and solved again this way.
 #include "gn_search.hpp"
 #include "invert_common.hpp"
@@ -24,7 +24,6 @@
 namespace gn {
 
 constexpr int kLeafIter = 8;  // projected Newton steps inside one leaf cell
-constexpr int kCand = 8;      // leaves collected per lane before the wave solves them
 
 // Whether a leaf can hold an interior foot point of P: a point X of its box b with P - X parallel
 // to a normal n of its cone (unit axis a, half-angle theta < 90 degrees), i.e. whether the box meets
@@ -34,7 +33,8 @@ constexpr int kCand = 8;      // leaves collected per lane before the wave solve
 // the line P + t a meets the box, or some edge has a point with q(s) >= 0, q being that quadratic
 // along the edge.  Exact up to rounding; FP64 on the FP32 box's bounds, with the half-angle widened
 // by another 2e-6 rad.
-__device__ __forceinline__ bool cone_may_hold(const float4 cn, const float *__restrict__ b,
+// c2: cos^2 of the widened half-angle, stored with the leaf's record at build time.
+__device__ __forceinline__ bool cone_may_hold(const float4 cn, double c2, const float (&b)[6],
                                               const double P[3]) {
     if (!(cn.w < 1.5f)) return true;  // no bounded cone
     const double a[3] = {cn.x, cn.y, cn.z};
@@ -54,7 +54,6 @@ __device__ __forceinline__ bool cone_may_hold(const float4 cn, const float *__re
         }
     }
     if (t0 <= t1) return true;  // also P inside the box (t = 0)
-    const double c = cos((double)cn.w + 2e-6), c2 = c * c;
     // the 12 edges: along axis k, the other two coordinates at their bounds
 #pragma unroll
     for (int k = 0; k < 3; k++) {
@@ -80,206 +79,477 @@ __device__ __forceinline__ bool cone_may_hold(const float4 cn, const float *__re
     return false;
 }
 
-// Projected Newton from (cu, cv) inside dom, with backtracking: a step after which the squared
+// Projected Newton with backtracking, one evaluation per call: a step after which the squared
 // distance grew by more than 1e-6 relative is halved, up to kHalvings times in a row, before a new
 // step is taken.  (Near a minimum the squared distance carries rounding of the surface point
-// relative to the residual, ~1e-12 of it at a 1e-3 offset; smaller growth is not a failed step.)
-// Returns the status and leaves in (cu, cv), d2 the nearest point evaluated and its squared
-// distance.  Inlined at its three call sites: as a called function its live values spilled
-// across the call (256 VGPRs + 224 bytes of scratch per lane, one wave per SIMD); inlined the
-// bicubic kernel takes 233 VGPRs, no scratch, two waves per SIMD (1M queries: 25.8 -> 7.7 ms).
+// relative to the residual, ~1e-12 of it at a 1e-3 offset; smaller growth is not a failed step.)  Once
+// the steps are over (`left` used up, or a final status) one more evaluation gives the distance of the
+// last iterate, and the nearer of it and the last accepted point is the solve's result.
 constexpr int kHalvings = 8;
-template <int K1, int K2, bool EXACT>
-__device__ __forceinline__ int solve_in(const GnSurfDev &d, const double *P, double &cu,
-                                        double &cv, const Domain &dom, int iters,
-                                        double tol_step, double &d2) {
-    SpanCache sc;
-    int st = GN_PT_MAXITER, back = 0;
-    double pu = cu, pv = cv, prr = INFINITY;  // the last accepted point
-    for (int it = 0; it < iters; it++) {
-        const double su = cu, sv = cv;
-        double rr = INFINITY;
-        const int s = gn_step<K1, K2, EXACT, double, true, kPatchGlobal, true>(
-            d, d.ku, d.kv, P[0], P[1], P[2], cu, cv, 0.0, tol_step, 0.0, 1, dom, sc, nullptr,
-            nullptr, &rr);
-        if (!(rr <= prr * (1.0 + 1e-6)) && back < kHalvings) {  // grew, beyond rounding
-            cu = pu + 0.5 * (su - pu);
-            cv = pv + 0.5 * (sv - pv);
-            back++;
-            continue;
-        }
+struct Solve {
+    double cu, cv;        // the iterate
+    double pu, pv, prr;   // the last accepted point and its squared distance
+    int left, back, st;   // steps left; halvings in a row; status (kStepContinue while stepping)
+    __device__ __forceinline__ void start(double u, double v, int iters) {
+        cu = pu = u;
+        cv = pv = v;
+        prr = INFINITY;
+        left = iters;
         back = 0;
-        pu = su;
-        pv = sv;
-        prr = rr;
-        if (s != kStepContinue) {
-            st = s;
-            break;
-        }
+        st = kStepContinue;
     }
-    Cart<double> o;
-    eval_point<K1, K2, 0, EXACT, double>(d, d.ku, d.kv, cu, cv, o);
-    const double dx = o.S[0] - P[0], dy = o.S[1] - P[1], dz = o.S[2] - P[2];
-    d2 = fma(dz, dz, fma(dy, dy, dx * dx));
-    if (!(d2 <= prr)) {  // the final step did not help: keep the last accepted point
-        cu = pu;
-        cv = pv;
-        d2 = prr;
-    }
-    return st;
-}
-
-// The branch and bound for query i.  Global mode (counts): also writes the number of leaves
-// solved to it32.  Fallback (!counts): the (u, v) already in place is kept when it is nearer.
-// cand: the workgroup's LDS candidate slots, kCand per thread (blocks of 256 threads).
-template <int K1, int K2, bool EXACT>
-__device__ __forceinline__ void project_point(const GnSurfDev &d, const GnSearchDev &sd,
-                                              const InvArgs &a, size_t i, bool counts,
-                                              uint32_t *cand) {
-    const Domain full = domain_of(d);
-    const int D = sd.depth;
-    // leaf cells: the unit square's 2^D x 2^D cells mapped onto the knot domain, exactly as the
-    // tree lays out its nodes' uv rectangles
-    const double cell = 1.0 / (double)(1u << D);
-    const double wu = full.u1 - full.u0, wv = full.v1 - full.v0;
-    const int max_iter = a.o.max_iter;
-    const double tol_step = a.o.tol_step;
-    const double P[3] = {a.x[i], a.y[i], a.z[i]};
-    // the bound solve starts from the greedy leaf's stepped seed (step_seed: one Gauss-Newton
-    // step and two on the leaf's quadratic model), a few Newton iterations nearer than its centre
-    float4 cq;
-    const uint32_t c0 = greedy_leaf(sd, P, nullptr, 0, &cq);
-    double bu, bv, best;
-    step_seed(sd, c0, cq, P, bu, bv);
-    int bst = solve_in<K1, K2, EXACT>(d, P, bu, bv, full, max_iter, tol_step, best);
-    int ncand = 1;
-    // The bound solve stands for leaf c0's own solve only if it ended inside c0's cell; a solve
-    // that wandered off may have passed a nearer minimum in the cell, so c0 then stays a candidate.
-    bool c0_done;
-    {
-        const uint32_t ix = compact2(c0 >> 1), iy = compact2(c0);
-        c0_done = bu >= full.u0 + wu * (ix * cell) && bu <= full.u0 + wu * ((ix + 1) * cell) &&
-                  bv >= full.v0 + wv * (iy * cell) && bv <= full.v0 + wv * ((iy + 1) * cell);
-    }
-    if (D > 0) {
-        const float p[3] = {(float)P[0], (float)P[1], (float)P[2]};
-        // stackless depth-first walk (Morton-code successor), pruned by the current best.  The
-        // walk collects up to kCand leaves at a time into this lane's LDS slots, then the wave
-        // solves them in rounds, each lane its r-th leaf: lanes walk different paths, but they
-        // solve together.  A collected leaf is solved only if its box is still not farther than
-        // the best so far; a leaf box is never nearer than its ancestors' boxes, so exactly the
-        // leaves of a walk that solved each leaf as it reached it are solved, in the same order.
-        const uint32_t side = 1u << D;
-        uint32_t *cq = cand + threadIdx.x * kCand;
-        int l = 1;
-        uint32_t c = 0;
-        bool walking = true;
-        while (__any(walking)) {  // wave-uniform
-            int nq = 0;
-            while (walking && nq < kCand) {
-                const double lb = (double)box_d2(sd.box32 + (qoff(l) + c) * 6, p);
-                bool descend = false;
-                if (lb <= best) {
-                    if (l < D) {
-                        descend = true;
-                    } else if ((c != c0 || !c0_done) &&
-                               (!sd.cone32 || compact2(c >> 1) - 1u >= side - 2u ||
-                                compact2(c) - 1u >= side - 2u ||
-                                cone_may_hold(sd.cone32[c], sd.box32 + (qoff(l) + c) * 6, P))) {
-                        // (the two index tests pass the leaves on the domain boundary, ix or iy
-                        // 0 or side - 1, by unsigned wrap-around)
-                        cq[nq++] = c;
-                    }
-                }
-                if (descend) {
-                    c <<= 2;
-                    l++;
-                    continue;
-                }
-                while (l > 1 && (c & 3u) == 3u) {
-                    c >>= 2;
-                    l--;
-                }
-                if (l == 1 && (c & 3u) == 3u) {
-                    walking = false;
-                    break;
-                }
-                c++;
+    // o: the surface at (cu, cv).  True when the solve is over: (cu, cv), d2 and st are its result.
+    __device__ __forceinline__ bool advance(const GnSurfDev &d, const Cart<double> &o, const double *P,
+                                            const Domain &dom, double tol_step, const SpanCache &sc,
+                                            double &d2) {
+        if (left > 0 && st == kStepContinue) {
+            left--;
+            const double su = cu, sv = cv;
+            double rr = INFINITY;
+            const int s = gn_update<double, true, true>(d, o, P[0], P[1], P[2], cu, cv, 0.0, tol_step,
+                                                        0.0, 1, dom, sc, &rr);
+            if (!(rr <= prr * (1.0 + 1e-6)) && back < kHalvings) {  // grew, beyond rounding
+                cu = pu + 0.5 * (su - pu);
+                cv = pv + 0.5 * (sv - pv);
+                back++;
+            } else {
+                back = 0;
+                pu = su;
+                pv = sv;
+                prr = rr;
+                st = s;
             }
-            for (int r = 0; __any(r < nq); r++) {  // wave-uniform rounds
-                if (r >= nq) continue;
-                const uint32_t lc = cq[r];
-                if (!((double)box_d2(sd.box32 + (qoff(D) + lc) * 6, p) <= best)) continue;
-                const uint32_t ix = compact2(lc >> 1), iy = compact2(lc);
-                const Domain cr{full.u0 + wu * (ix * cell), full.u0 + wu * ((ix + 1) * cell),
-                                full.v0 + wv * (iy * cell), full.v0 + wv * ((iy + 1) * cell)};
-                // from the leaf's stepped seed for P (step_seed from its record), clamped into
-                // its cell: fewer Newton steps than from the cell centre
-                double cu, cv, d2;
-                step_seed(sd, lc, sd.rec[(size_t)lc * kRecVec], P, cu, cv);
-                cu = fmin(fmax(cu, cr.u0), cr.u1);
-                cv = fmin(fmax(cv, cr.v0), cr.v1);
-                const int s2 = solve_in<K1, K2, EXACT>(d, P, cu, cv, cr, kLeafIter, tol_step, d2);
-                ncand++;
-                if (d2 < best) {
-                    best = d2;
-                    bu = cu;
-                    bv = cv;
-                    bst = s2;
-                }
-            }
+            return false;
         }
-    }
-    double pu = bu, pv = bv, pd2;
-    const int pst = solve_in<K1, K2, EXACT>(d, P, pu, pv, full, max_iter, tol_step, pd2);
-    if (pd2 <= best * (1.0 + 1e-9)) {  // not farther beyond rounding: the polished point
-        bu = pu;
-        bv = pv;
-        bst = pst;
-        best = pd2;
-    }
-    if (!counts) {  // fallback: the earlier result stays if it is nearer
-        Cart<double> o;
-        eval_point<K1, K2, 0, EXACT, double>(d, d.ku, d.kv, a.u[i], a.v[i], o);
         const double dx = o.S[0] - P[0], dy = o.S[1] - P[1], dz = o.S[2] - P[2];
-        if (fma(dz, dz, fma(dy, dy, dx * dx)) < best) return;
+        d2 = fma(dz, dz, fma(dy, dy, dx * dx));
+        if (!(d2 <= prr)) {  // the final step did not help: keep the last accepted point
+            cu = pu;
+            cv = pv;
+            d2 = prr;
+        }
+        if (st == kStepContinue) st = GN_PT_MAXITER;
+        return true;
     }
-    a.u[i] = bu;
-    a.v[i] = bv;
-    a.status[i] = (uint8_t)bst;
-    if (counts) {
-        if (a.it32) a.it32[i] = sat8(ncand);
-        if (a.it64) a.it64[i] = 0;
-    }
-}
+};
 
 // Two waves per SIMD are forced where the spills that costs stay small: patches of up to 20
-// entries (bicubic: 12 bytes per lane; one wave without the bound, 13.3 against 8.2 ms on 1M
-// projection queries; degree (3,4): 160 bytes, 14.3 against 9.1 ms) and the generic kernel (80
-// bytes, 12.9 against 7.2 ms).  Larger exact patches run one wave with AGPRs as spill room:
-// forced to two, degree (5,5) spilled 744 bytes per lane and took 24.5 against 18.3 ms.
+// entries and the generic kernel.  Larger exact patches run one wave with AGPRs as spill room.
 template <int K1, int K2, bool EXACT>
 constexpr int project_waves() { return (!EXACT || K1 * K2 <= 20) ? 2 : 1; }
 
-// order (may be null): the queries in the order to take them, so that a wave's lanes hold
-// queries near one another in space and walk much the same part of the tree (k_proj_order).
-template <int K1, int K2, bool EXACT>
-__global__ __launch_bounds__(256, (project_waves<K1, K2, EXACT>())) void k_project_global(
-    GnSurfDev d, GnSearchDev sd, InvArgs a, const uint32_t *__restrict__ order) {
-    __shared__ uint32_t cand[256 * kCand];
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < a.n;
-         i += (size_t)gridDim.x * blockDim.x)
-        project_point<K1, K2, EXACT>(d, sd, a, order ? (size_t)order[i] : i, true, cand);
+// Levels of the seed quadtree whose FP32 boxes a workgroup stages in LDS: levels 1..4 are 340
+// boxes, 8 KB.
+constexpr int kProjLdsLevels = 4;
+
+// The largest float not above x: a float is <= x exactly when it is <= floor32(x).
+__device__ __forceinline__ float floor32(double x) { return __double2float_rd(x); }
+
+// N consecutive boxes (6 floats each): the mask of those not farther than best32.
+template <int N, typename PTR>
+__device__ __forceinline__ uint32_t box_mask(PTR boxes, const float p[3], float best32) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int k = 0; k < N; k++) {
+        float b[6];
+        __builtin_memcpy(b, boxes + 6 * k, sizeof(b));
+        if (box_d2(b, p) <= best32) m |= 1u << k;
+    }
+    return m;
+}
+
+// The branch and bound over a wave's chunk of up to kProjQ consecutive queries (grid-stride), its state
+// in LDS.  The wave alternates between two kinds of phases:
+//   - lane per query: the queries' starts; walks of the tree (Morton order, so the same leaves in the
+//     same order as a walk that solved each leaf on arrival) that collect the next leaves to solve into
+//     a pool of kProjItems; the choice among solved leaves; the results;
+//   - lane per solve: the bound solves, the pool's leaf solves, the polishes.  Lanes take the next
+//     solve of the phase as they finish, and a query's leaves are solved by several lanes at once.
+// A collected leaf counts only if its box is not farther than the best point so far when its turn
+// comes in the query's order; a leaf whose box is farther cannot hold a nearer point, so solving it
+// ahead of its turn changes no result.
+// What bounds the kernel is FP64 evaluation (one step of up to 64 solves: 2.9 us per wave at two waves
+// per SIMD, 40 lanes active on average) and then the walks, about a fifth; for small calls the longest
+// chain of solves.  One query per lane, its solves gathered into rounds with the other lanes', kept 19%
+// of the lanes active: 262,144 queries on a bicubic 32 x 32 net took 1199 us and now take 490, 1,000
+// queries 463 and 133 us.  One wave per SIMD without spills (273 registers): 696 us.
+// LIST: the fallback over list[0 .. *count): the (u, v) already in place is kept when it is nearer, and
+// the counts are left alone.  Otherwise it32 receives the number of leaves solved.
+constexpr int kProjQ = 128, kProjItems = 224, kProjPer = 6;
+struct ProjWave {
+    double P[3][kProjQ];
+    double best[kProjQ], bu[kProjQ], bv[kProjQ];
+    // per tree level, 4 bits: passing children not yet visited; at level depth - 2, 16 bits: leaves
+    unsigned long long stack[kProjQ];
+    uint32_t c0[kProjQ], path[kProjQ];
+    uint16_t solved[kProjQ];
+    uint8_t level[kProjQ], bst[kProjQ];
+    uint8_t first[kProjQ], taken[kProjQ];  // the query's places in the pool
+    // the pool: query, leaf, box distance; start, then result
+    union {
+        struct {
+            double iu[kProjItems], iv[kProjItems], id2[kProjItems];
+        };
+        struct {  // while the pool is filled: the leaves the walks found, and which may hold a foot point
+            uint32_t found[kProjQ][kProjPer];
+            uint16_t cand[kProjQ * kProjPer];
+            uint32_t holds[kProjQ];
+        };
+    };
+    uint32_t ileaf[kProjItems];
+    float ilb[kProjItems];
+    uint8_t iq[kProjItems], ist[kProjItems];
+};
+static_assert(kProjItems <= 256 && kProjPer <= 8, "pool places and leaf counts are bytes");
+enum { kProjBound = 0, kProjLeaves = 1, kProjPolish = 2 };
+
+__device__ __forceinline__ void wave_lds_order() {  // LDS accesses before stay before, across lanes
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int K1, int K2, bool EXACT, bool LIST>
+__global__ __launch_bounds__(256, (project_waves<K1, K2, EXACT>())) void k_project(
+    GnSurfDev d_in, GnSearchDev sd, InvArgs a, const uint32_t *__restrict__ order,
+    const uint32_t *__restrict__ count, int chunk) {
+    extern __shared__ double sk[];  // EXACT: knots and reciprocal span lengths
+    __shared__ __align__(16) float lbox[(((1 << (2 * (kProjLdsLevels + 1))) - 1) / 3 - 1) * 6];
+    __shared__ ProjWave waves[4];
+    const int D = sd.depth, ll = D < kProjLdsLevels ? D : kProjLdsLevels;
+    {
+        const int nf2 = (int)(qoff(ll + 1) - 1) * 3;
+        const float2 *src = reinterpret_cast<const float2 *>(sd.box32 + 6);
+        float2 *dst = reinterpret_cast<float2 *>(lbox);
+        for (int i = threadIdx.x; i < nf2; i += blockDim.x) dst[i] = src[i];
+    }
+    GnSurfDev d = d_in;
+    const double *ku = d_in.ku, *kv = d_in.kv;
+    if constexpr (EXACT) {  // (also waits for the boxes)
+        d = stage_knots_lds(d_in, sk);
+        ku = sk;
+        kv = sk + d.nu + d.p + 1;
+    } else {
+        __syncthreads();
+    }
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    ProjWave &w = waves[wv];
+    const unsigned long long lt = (1ull << lane) - 1ull;
+    const Domain full{ku[d.p], ku[d.nu], kv[d.q], kv[d.nv]};
+    const uint32_t side = 1u << D;
+    // leaf cells: the unit square's 2^D x 2^D cells mapped onto the knot domain, exactly as the
+    // tree lays out its nodes' uv rectangles
+    const double cell = 1.0 / (double)side;
+    const double wu = full.u1 - full.u0, wvv = full.v1 - full.v0;
+    auto leaf_cell = [&](uint32_t c) __attribute__((always_inline)) {
+        const uint32_t ix = compact2(c >> 1), iy = compact2(c);
+        return Domain{full.u0 + wu * (ix * cell), full.u0 + wu * ((ix + 1) * cell),
+                      full.v0 + wvv * (iy * cell), full.v0 + wvv * ((iy + 1) * cell)};
+    };
+    const int max_iter = a.o.max_iter;
+    const double tol_step = a.o.tol_step;
+    const size_t n = LIST ? (size_t)*count : a.n;
+    for (size_t q0 = ((size_t)blockIdx.x * 4 + wv) * (size_t)chunk; q0 < n;
+         q0 += (size_t)gridDim.x * 4 * (size_t)chunk) {  // wave-uniform
+        const int nq = (int)(n - q0 < (size_t)chunk ? n - q0 : (size_t)chunk);
+        // starts: the greedy leaf's stepped seed (step_seed: one Gauss-Newton step and two on the
+        // leaf's quadratic model), a few Newton iterations nearer than its centre
+        for (int q = lane; q < nq; q += 64) {
+            const size_t i = LIST || order ? (size_t)order[q0 + q] : q0 + q;
+            const double P[3] = {a.x[i], a.y[i], a.z[i]};
+            float4 cq;
+            const uint32_t c0 = greedy_leaf(sd, P, lbox, ll, &cq);
+            double bu, bv;
+            step_seed(sd, c0, cq, P, bu, bv);
+            w.P[0][q] = P[0];
+            w.P[1][q] = P[1];
+            w.P[2][q] = P[2];
+            w.bu[q] = bu;
+            w.bv[q] = bv;
+            w.c0[q] = c0;
+            w.solved[q] = 1;
+        }
+        int phase = kProjBound, items = nq;  // wave-uniform
+        while (true) {
+            // ---- a lane per solve
+            wave_lds_order();
+            {
+                int next = 0, it = 0;
+                bool act = false;
+                Solve sv;
+                sv.start(full.u0, full.v0, 0);
+                SpanCache sc;
+                Domain dom = full;
+                double P[3] = {0, 0, 0};
+                while (true) {
+                    const unsigned long long idle = __ballot(!act);
+                    if (idle && next < items) {
+                        const int rank = __popcll(idle & lt);
+                        if (!act && rank < items - next) {
+                            it = next + rank;
+                            int q = it;
+                            double su, s_v;
+                            if (phase == kProjLeaves) {
+                                q = w.iq[it];
+                                su = w.iu[it];
+                                s_v = w.iv[it];
+                                dom = leaf_cell(w.ileaf[it]);
+                            } else {
+                                su = w.bu[it];
+                                s_v = w.bv[it];
+                                dom = full;
+                            }
+                            P[0] = w.P[0][q];
+                            P[1] = w.P[1][q];
+                            P[2] = w.P[2][q];
+                            sv.start(su, s_v, phase == kProjLeaves ? kLeafIter : max_iter);
+                            act = true;
+                        }
+                        const int took = __popcll(idle);
+                        next += took < items - next ? took : items - next;
+                    }
+                    if (!__any(act)) break;
+                    if (act) {
+                        Cart<double> o;
+                        eval_point_cached<K1, K2, 2, EXACT, double, kPatchGlobal, true>(
+                            d, ku, kv, sv.cu, sv.cv, sc, o);
+                        double d2;
+                        if (sv.advance(d, o, P, dom, tol_step, sc, d2)) {
+                            act = false;
+                            if (phase == kProjLeaves) {
+                                w.iu[it] = sv.cu;
+                                w.iv[it] = sv.cv;
+                                w.id2[it] = d2;
+                                w.ist[it] = (uint8_t)sv.st;
+                            } else if (phase == kProjBound || d2 <= w.best[it] * (1.0 + 1e-9)) {
+                                // the bound; or the polished point, if not farther beyond rounding
+                                w.best[it] = d2;
+                                w.bu[it] = sv.cu;
+                                w.bv[it] = sv.cv;
+                                w.bst[it] = (uint8_t)sv.st;
+                            }
+                        }
+                    }
+                }
+            }
+            wave_lds_order();
+            if (phase == kProjPolish) break;
+            // ---- a lane per query: the best of the leaves solved, in the query's order
+            for (int q = lane; q < nq; q += 64) {
+                const float p[3] = {(float)w.P[0][q], (float)w.P[1][q], (float)w.P[2][q]};
+                if (phase == kProjBound) {
+                    // the root's children (a tree of one leaf has nothing to walk)
+                    unsigned long long stk = 0;
+                    if (D > 0) stk = box_mask<4>(lbox, p, floor32(w.best[q]));
+                    w.stack[q] = stk;
+                    w.path[q] = 0;
+                    w.level[q] = 0;
+                    // The bound solve stands for leaf c0's own solve only if it ended inside c0's
+                    // cell; a solve that wandered off may have passed a nearer minimum in the
+                    // cell, so c0 then stays a candidate (no leaf is left out).
+                    const uint32_t c0 = w.c0[q];
+                    const Domain cr = leaf_cell(c0);
+                    const double bu = w.bu[q], bv = w.bv[q];
+                    if (!(bu >= cr.u0 && bu <= cr.u1 && bv >= cr.v0 && bv <= cr.v1)) w.c0[q] = 0xffffffffu;
+                } else {
+                    double best = w.best[q];
+                    const int i0 = w.first[q], i1 = i0 + w.taken[q];
+                    for (int i = i0; i < i1; i++) {
+                        if (!((double)w.ilb[i] <= best)) continue;
+                        w.solved[q] += w.solved[q] < 0xffffu;
+                        if (w.id2[i] < best) {
+                            best = w.id2[i];
+                            w.bu[q] = w.iu[i];
+                            w.bv[q] = w.iv[i];
+                            w.bst[q] = w.ist[i];
+                        }
+                    }
+                    w.best[q] = best;
+                }
+            }
+            wave_lds_order();
+            // ---- the queries' walks: up to kProjPer leaves each, from where the last walk stopped
+            unsigned long long stk[kProjQ / 64];
+            uint32_t path[kProjQ / 64];
+            int level[kProjQ / 64], nf[kProjQ / 64];
+            int cands = 0;  // wave-uniform
+#pragma unroll
+            for (int g = 0; g < kProjQ / 64; g++) {
+                const int q = 64 * g + lane, qs = q < nq ? q : 0;
+                stk[g] = q < nq ? w.stack[qs] : 0ull;
+                path[g] = w.path[qs];
+                level[g] = w.level[qs];
+                nf[g] = 0;
+                if (__any(stk[g] != 0)) {
+                    const float p[3] = {(float)w.P[0][qs], (float)w.P[1][qs], (float)w.P[2][qs]};
+                    const float best32 = floor32(w.best[qs]);
+                    const uint32_t c0 = w.c0[qs];
+                    unsigned long long sk_ = stk[g];
+                    uint32_t c = path[g];
+                    int l = level[g], k = 0;
+                    bool look = sk_ != 0;
+                    while (look) {
+                        const bool low = l == D - 2;  // a node whose 16 leaves are left
+                        const uint32_t m = (uint32_t)(sk_ >> (4 * l)) & (low ? 0xffffu : 15u);
+                        if (!m) {
+                            if (l == 0) break;
+                            c >>= 2;
+                            l--;
+                            continue;
+                        }
+                        const int j = __ffs(m) - 1;
+                        sk_ &= ~(1ull << (4 * l + j));
+                        if (low) {
+                            if (16 * c + j == c0) continue;
+                            w.found[q][k++] = 16 * c + j;
+                            look = k < kProjPer;
+                            continue;
+                        }
+                        c = 4 * c + j;
+                        l++;
+                        uint32_t cm;
+                        if (l == D - 2) cm = box_mask<16>(sd.box32 + (qoff(D) + 16 * c) * 6, p, best32);
+                        else if (l < ll) cm = box_mask<4>(lbox + (qoff(l + 1) - 1 + 4 * c) * 6, p, best32);
+                        else cm = box_mask<4>(sd.box32 + (qoff(l + 1) + 4 * c) * 6, p, best32);
+                        sk_ |= (unsigned long long)cm << (4 * l);
+                    }
+                    stk[g] = sk_;
+                    path[g] = c;
+                    level[g] = l;
+                    nf[g] = k;
+                }
+                // the candidates of all queries, one list
+                if (q < nq) w.holds[q] = 0u;
+                for (int k = 0; __any(nf[g] > k); k++) {
+                    const unsigned long long m = __ballot(nf[g] > k);
+                    if (nf[g] > k) w.cand[cands + __popcll(m & lt)] = (uint16_t)(q * 8 + k);
+                    cands += __popcll(m);
+                }
+            }
+            wave_lds_order();
+            // a lane per candidate: may the leaf hold a nearer foot point?  (The bound may have fallen
+            // since its box was tested; the two index tests pass the leaves on the domain boundary, ix
+            // or iy 0 or side - 1, by unsigned wrap-around.)
+            for (int e = lane; e < cands; e += 64) {
+                const int q = w.cand[e] >> 3, k = w.cand[e] & 7;
+                const uint32_t leaf = w.found[q][k];
+                const double P[3] = {w.P[0][q], w.P[1][q], w.P[2][q]};
+                const float p[3] = {(float)P[0], (float)P[1], (float)P[2]};
+                float b[6];
+                __builtin_memcpy(b, sd.box32 + (qoff(D) + leaf) * 6, sizeof(b));
+                if (box_d2(b, p) <= floor32(w.best[q]) &&
+                    (!sd.cone32 || compact2(leaf >> 1) - 1u >= side - 2u ||
+                     compact2(leaf) - 1u >= side - 2u ||
+                     cone_may_hold(sd.cone32[leaf],
+                                   *reinterpret_cast<const double *>(sd.rec + (size_t)leaf * kRecVec + 7),
+                                   b, P)))
+                    __hip_atomic_fetch_or(&w.holds[q], 1u << k, __ATOMIC_RELAXED,
+                                          __HIP_MEMORY_SCOPE_WAVEFRONT);
+            }
+            wave_lds_order();
+            // into the pool, queries in order while there is room for all of a query's leaves (the
+            // others walk again next time)
+            items = 0;
+#pragma unroll
+            for (int g = 0; g < kProjQ / 64; g++) {
+                const int q = 64 * g + lane;
+                const uint32_t h = q < nq ? w.holds[q] : 0u;
+                const int cnt = __popc(h);
+                int end = cnt;  // inclusive prefix sum over the wave
+#pragma unroll
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int x = __shfl_up(end, o, 64);
+                    if (lane >= o) end += x;
+                }
+                const bool fits = items + end <= kProjItems;
+                int at = items + end - cnt;
+                if (q < nq) {
+                    w.first[q] = (uint8_t)at;
+                    w.taken[q] = (uint8_t)(fits ? cnt : 0);
+                    if (fits) {
+                        w.stack[q] = stk[g];
+                        w.path[q] = path[g];
+                        w.level[q] = (uint8_t)level[g];
+                        for (uint32_t m = h; m; m &= m - 1) {
+                            w.ileaf[at] = w.found[q][__ffs(m) - 1];
+                            w.iq[at++] = (uint8_t)q;
+                        }
+                    }
+                }
+                const unsigned long long fm = __ballot(fits);
+                // prefix sums do not fall, so the fitting lanes are a leading run
+                const int last = __popcll(fm) - 1;
+                items += last >= 0 ? __shfl(end, last < 0 ? 0 : last, 64) : 0;
+                if (fm != ~0ull) {  // later groups wait too
+#pragma unroll
+                    for (int g2 = g + 1; g2 < kProjQ / 64; g2++) {
+                        const int q2 = 64 * g2 + lane;
+                        if (q2 < nq) w.taken[q2] = 0;
+                    }
+                    break;
+                }
+            }
+            wave_lds_order();
+            // a lane per leaf: its start, the leaf's stepped seed for P clamped into its cell (fewer
+            // Newton steps than from the cell centre)
+            for (int i = lane; i < items; i += 64) {
+                const int q = w.iq[i];
+                const uint32_t leaf = w.ileaf[i];
+                const double P[3] = {w.P[0][q], w.P[1][q], w.P[2][q]};
+                const float p[3] = {(float)P[0], (float)P[1], (float)P[2]};
+                float b[6];
+                __builtin_memcpy(b, sd.box32 + (qoff(D) + leaf) * 6, sizeof(b));
+                const Domain cr = leaf_cell(leaf);
+                double cu, cv;
+                step_seed(sd, leaf, sd.rec[(size_t)leaf * kRecVec], P, cu, cv);
+                w.ilb[i] = box_d2(b, p);
+                w.iu[i] = fmin(fmax(cu, cr.u0), cr.u1);
+                w.iv[i] = fmin(fmax(cv, cr.v0), cr.v1);
+            }
+            // nothing in the pool, and every walk at its end: the polish
+            phase = kProjLeaves;
+            if (!items) {
+                bool left = false;
+                for (int q = lane; q < nq; q += 64) left |= w.stack[q] != 0;
+                if (!__any(left)) {
+                    phase = kProjPolish;
+                    items = nq;
+                }
+            }
+        }
+        // ---- results
+        for (int q = lane; q < nq; q += 64) {
+            const size_t i = LIST || order ? (size_t)order[q0 + q] : q0 + q;
+            if constexpr (LIST) {  // the earlier result stays if it is nearer
+                Cart<double> e;
+                eval_point<K1, K2, 0, EXACT, double>(d, ku, kv, a.u[i], a.v[i], e);
+                const double dx = e.S[0] - w.P[0][q], dy = e.S[1] - w.P[1][q], dz = e.S[2] - w.P[2][q];
+                if (fma(dz, dz, fma(dy, dy, dx * dx)) < w.best[q]) continue;
+            }
+            a.u[i] = w.bu[q];
+            a.v[i] = w.bv[q];
+            a.status[i] = w.bst[q];
+            if constexpr (!LIST) {
+                if (a.it32) a.it32[i] = sat8(w.solved[q]);
+                if (a.it64) a.it64[i] = 0;
+            }
+        }
+        wave_lds_order();
+    }
 }
 
 // Spatial order of the queries: the key is the 16 x 16 x 16 cell of P within the tree's root box
 // (Morton order, 12 bits; points outside the box take its border cells, NaN coordinates cell 0).
 // One workgroup per block of kOrdBlock consecutive queries counts its keys in LDS, scans them and
-// writes each query's index to its key's next slot within the block's own range of `order`.  The
+// writes each query's index to its key's next slot within the block's own range of `order`.  Keys stay
+// in registers between the two passes and the block's loads are issued together: with blocks of 65,536
+// read twice in sequence, four workgroups took 103 us for 262,144 queries.  The
 // order within one key is unspecified; each query's result does not depend on it (project_point
 // is per query).
 constexpr int kOrdThreads = 1024;
-constexpr size_t kOrdBlock = 65536;
+constexpr int kOrdPer = 16;  // queries per thread
+constexpr size_t kOrdBlock = (size_t)kOrdPer * kOrdThreads;
 constexpr int kOrdKeys = 4096;
 
 __device__ __forceinline__ uint32_t proj_key(const float *__restrict__ root, const double P[3]) {
@@ -309,10 +579,17 @@ __global__ __launch_bounds__(kOrdThreads) void k_proj_order(const float *__restr
     __syncthreads();
     const size_t i0 = (size_t)blockIdx.x * kOrdBlock;
     const size_t i1 = i0 + kOrdBlock < n ? i0 + kOrdBlock : n;
-    for (size_t i = i0 + threadIdx.x; i < i1; i += kOrdThreads) {
-        const double P[3] = {x[i], y[i], z[i]};
-        atomicAdd(&cnt[proj_key(root, P)], 1u);
+    uint32_t key[kOrdPer];
+#pragma unroll
+    for (int k = 0; k < kOrdPer; k++) {
+        const size_t i = i0 + (size_t)k * kOrdThreads + threadIdx.x;
+        const size_t j = i < i1 ? i : i1 - 1;
+        const double P[3] = {x[j], y[j], z[j]};
+        key[k] = proj_key(root, P);
     }
+#pragma unroll
+    for (int k = 0; k < kOrdPer; k++)
+        if (i0 + (size_t)k * kOrdThreads + threadIdx.x < i1) atomicAdd(&cnt[key[k]], 1u);
     __syncthreads();
     // exclusive scan: each thread a run of kOrdKeys / kOrdThreads keys, then the runs' sums
     constexpr int per = kOrdKeys / kOrdThreads;
@@ -336,22 +613,11 @@ __global__ __launch_bounds__(kOrdThreads) void k_proj_order(const float *__restr
         run += c;
     }
     __syncthreads();
-    for (size_t i = i0 + threadIdx.x; i < i1; i += kOrdThreads) {
-        const double P[3] = {x[i], y[i], z[i]};
-        order[atomicAdd(&cnt[proj_key(root, P)], 1u)] = (uint32_t)i;
+#pragma unroll
+    for (int k = 0; k < kOrdPer; k++) {
+        const size_t i = i0 + (size_t)k * kOrdThreads + threadIdx.x;
+        if (i < i1) order[atomicAdd(&cnt[key[k]], 1u)] = (uint32_t)i;
     }
-}
-
-// The fallback: the queries listed in list[0 .. *count) (iteration counts left as they were).
-template <int K1, int K2, bool EXACT>
-__global__ __launch_bounds__(256) void k_project_list(GnSurfDev d, GnSearchDev sd, InvArgs a,
-                                                      const uint32_t *__restrict__ list,
-                                                      const uint32_t *__restrict__ count) {
-    __shared__ uint32_t cand[256 * kCand];
-    const size_t cnt = *count;
-    for (size_t j = (size_t)blockIdx.x * blockDim.x + threadIdx.x; j < cnt;
-         j += (size_t)gridDim.x * blockDim.x)
-        project_point<K1, K2, EXACT>(d, sd, a, list[j], false, cand);
 }
 
 __global__ void k_fb_zero(uint32_t *count) { *count = 0u; }
@@ -365,16 +631,27 @@ __global__ void k_fb_compact(const uint8_t *__restrict__ status, size_t n, uint3
             list[atomicAdd(count, 1u)] = (uint32_t)i;
 }
 
+// Queries per wave chunk: a full pool's worth (kProjQ) once that still gives every resident wave (two
+// per SIMD) a chunk, fewer for smaller calls, whose time is the longest chain of solves in a wave.
+inline int project_chunk(size_t n) {
+    const size_t waves = (size_t)cu_count() * 8;
+    size_t c = (n / waves + 15) / 16 * 16;
+    return (int)(c < 16 ? 16 : c > (size_t)kProjQ ? (size_t)kProjQ : c);
+}
+
 struct ProjectLaunch {
     const GnSurfDev &d;
     const GnSearchDev &sd;
     const InvArgs &a;
-    const uint32_t *order;
+    const uint32_t *order, *count;  // count: the fallback's list length
     hipStream_t st;
     template <int K1, int K2, bool EXACT>
     int operator()() {
-        k_project_global<K1, K2, EXACT><<<grid_for(a.n, 256, 256 * 16), 256, 0, st>>>(d, sd, a,
-                                                                                    order);
+        const int chunk = count ? 16 : project_chunk(a.n);
+        const unsigned grid = grid_for(a.n, 4 * chunk, 1u << 24);
+        const size_t lds = EXACT ? sizeof(double) * (2 * d.nu + 2 * d.nv + 2) : 0;
+        if (count) k_project<K1, K2, EXACT, true><<<grid, 256, lds, st>>>(d, sd, a, order, count, chunk);
+        else k_project<K1, K2, EXACT, false><<<grid, 256, lds, st>>>(d, sd, a, order, nullptr, chunk);
         GN_HIP(hipGetLastError());
         return GN_OK;
     }
@@ -398,25 +675,10 @@ int launch_project_global(const GnSurfDev &d, const GnSearchDev &sd, const InvAr
             return fail(GN_EDEVICE, "query ordering launch");
         }
     }
-    const int rc = dispatch_degrees(d.p, d.q, ProjectLaunch{d, sd, a, order, st});
+    const int rc = dispatch_inv(d, ProjectLaunch{d, sd, a, order, nullptr, st});
     if (order) GN_HIP(hipFreeAsync(order, st));
     return rc;
 }
-
-struct ListLaunch {
-    const GnSurfDev &d;
-    const GnSearchDev &sd;
-    const InvArgs &a;
-    const uint32_t *list, *count;
-    hipStream_t st;
-    template <int K1, int K2, bool EXACT>
-    int operator()() {
-        k_project_list<K1, K2, EXACT><<<grid_for(a.n, 256, 256 * 16), 256, 0, st>>>(d, sd, a, list,
-                                                                                 count);
-        GN_HIP(hipGetLastError());
-        return GN_OK;
-    }
-};
 
 // After an inversion on st: the unconverged queries are listed on the device (stream-ordered
 // scratch of n + 1 words) and solved again by the global projection.
@@ -430,7 +692,7 @@ int launch_project_fallback(const GnSurfDev &d, const GnSearchDev &sd, const Inv
     k_fb_zero<<<1, 1, 0, st>>>(count);
     k_fb_compact<<<grid_for(a.n, 256, 256 * 16), 256, 0, st>>>(a.status, a.n, list, count);
     int rc = hipGetLastError() == hipSuccess ? GN_OK : fail(GN_EDEVICE, "fallback compaction launch");
-    if (!rc) rc = dispatch_degrees(d.p, d.q, ListLaunch{d, sd, a, list, count, st});
+    if (!rc) rc = dispatch_inv(d, ProjectLaunch{d, sd, a, list, count, st});
     GN_HIP(hipFreeAsync(buf, st));
     return rc;
 }

@@ -218,7 +218,7 @@ __global__ void k_search_box32(long total, const double *__restrict__ sbox,
 }
 
 // S_u, S_v, S_uu, S_uv, S_vv at every leaf's seed (u, v), for the stepped seeds: one thread per
-// leaf, into vectors 2..6 of the leaf's record (7 zero).
+// leaf, into vectors 2..6 of the leaf's record (7 is the cone's, k_search_cone).
 template <int K1, int K2, bool EXACT>
 __global__ void k_search_jac(GnSurfDev d, long leaves, const double *__restrict__ sseed,
                              float4 *__restrict__ srec) {
@@ -229,7 +229,7 @@ __global__ void k_search_jac(GnSurfDev d, long leaves, const double *__restrict_
     const double *f[5] = {o.Su, o.Sv, o.Suu, o.Suv, o.Svv};
     float4 *r = srec + c * kRecVec;
     for (int k = 0; k < 5; k++) r[2 + k] = make_float4((float)f[k][0], (float)f[k][1], (float)f[k][2], 0.f);
-    r[7] = make_float4(0.f, 0.f, 0.f, 0.f);
+    r[7] = make_float4(0.f, 0.f, 0.f, 0.f);  // k_search_cone fills its first half
 }
 
 // Normal cone of every leaf (NormalBoundingBox + NormalBoxToNormalTreeNode,
@@ -248,7 +248,8 @@ __device__ __forceinline__ void cross3(const double *a, const double *b, double 
 
 template <int K1, int K2, bool EXACT>
 __global__ __launch_bounds__(64) void k_search_cone(GnSurfDev d, int levels,
-                                                    float4 *__restrict__ cone32) {
+                                                    float4 *__restrict__ cone32,
+                                                    float4 *__restrict__ srec) {
     long g = 1;
     for (int l = 1; l < levels; l++) g *= 8;
     const long idx = blockIdx.x;  // bx * g + by
@@ -321,19 +322,23 @@ __global__ __launch_bounds__(64) void k_search_cone(GnSurfDev d, int levels,
         if ((double)t32 < th + 1e-6) t32 = nextafterf(t32, INFINITY);
         out = make_float4((float)(m[0] / mm), (float)(m[1] / mm), (float)(m[2] / mm), t32);
     }
-    cone32[morton2((uint32_t)bx, (uint32_t)by)] = out;
+    const uint32_t c = morton2((uint32_t)bx, (uint32_t)by);
+    cone32[c] = out;
+    // cos^2 of the half-angle widened by 2e-6 rad (cone_may_hold), in the leaf record's last vector
+    const double cw = cos((double)out.w + 2e-6);
+    *reinterpret_cast<double *>(srec + (size_t)c * kRecVec + 7) = cw * cw;
 }
 
 struct ConeLaunch {
     const GnSurfDev &d;
     int levels;
-    float4 *cone32;
+    float4 *cone32, *srec;
     hipStream_t st;
     template <int K1, int K2, bool EXACT>
     int operator()() {
         long g = 1;
         for (int l = 1; l < levels; l++) g *= 8;
-        k_search_cone<K1, K2, EXACT><<<(unsigned)(g * g), 64, 0, st>>>(d, levels, cone32);
+        k_search_cone<K1, K2, EXACT><<<(unsigned)(g * g), 64, 0, st>>>(d, levels, cone32, srec);
         GN_HIP(hipGetLastError());
         return GN_OK;
     }
@@ -363,7 +368,7 @@ int launch_search_build(const GnSurfDev &d, int levels, const GnTreeNode *tree, 
                                                                        sseed, sref, sleaf32, srec);
     GN_HIP(hipGetLastError());
     int rc = dispatch_degrees(d.p, d.q, JacLaunch{d, leaves, sseed, srec, st});
-    if (!rc) rc = dispatch_degrees(d.p, d.q, ConeLaunch{d, levels, scone32, st});
+    if (!rc) rc = dispatch_degrees(d.p, d.q, ConeLaunch{d, levels, scone32, srec, st});
     if (rc) return rc;
     for (int l = D - 1; l >= 0; l--)
         k_search_level<<<grid_for(1L << (2 * l), 256, 1u << 30), 256, 0, st>>>(l, sbox);

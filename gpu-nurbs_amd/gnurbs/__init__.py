@@ -149,18 +149,32 @@ def _check(rc: int):
         raise GnError(rc, lib().gn_last_error().decode())
 
 
-def _torch():
-    import torch
+_ready = None  # torch, once a GPU has been seen
 
-    if not torch.cuda.is_available():
-        raise RuntimeError("gnurbs needs a visible GPU (HIP device); none is available")
-    return torch
+
+def _torch():
+    global _ready
+    if _ready is None:
+        import torch
+
+        if not torch.cuda.is_available():
+            raise RuntimeError("gnurbs needs a visible GPU (HIP device); none is available")
+        torch.cuda.init()
+        _ready = torch
+    return _ready
 
 
 def stream_handle(stream=None) -> int:
     torch = _torch()
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    return _raw_stream(torch.cuda.current_device())
+
+
+def _raw_stream(device: int) -> int:
+    # the current stream's handle without building a Stream object, which costs as much as a launch
+    get = getattr(_ready._C, "_cuda_getCurrentRawStream", None)
+    return get(device) if get is not None else _ready.cuda.current_stream().cuda_stream
 
 
 def to_device(x, dtype):
@@ -168,6 +182,8 @@ def to_device(x, dtype):
     torch = _torch()
     if isinstance(x, np.ndarray):
         x = torch.from_numpy(np.ascontiguousarray(x))
+    elif x.is_cuda and x.dtype is dtype and x.get_device() == torch.cuda.current_device() and x.is_contiguous():
+        return x
     return x.to(device="cuda", dtype=dtype).contiguous()
 
 
@@ -218,7 +234,7 @@ class Surface:
             nu, nv = w.shape
             h = _c_void()
             _check(lib().gn_surface_create(int(degree_u), int(degree_v), nu, nv, ku.ctypes.data, kv.ctypes.data,
-                                           cp.ctypes.data, w.ctypes.data, _c_void(stream_handle(stream)), ctypes.byref(h)))
+                                           cp.ctypes.data, w.ctypes.data, stream_handle(stream), ctypes.byref(h)))
             self._h = h
         p, q, nu, nv = _c_int(), _c_int(), _c_int(), _c_int()
         _check(lib().gn_surface_info(self._h, ctypes.byref(p), ctypes.byref(q), ctypes.byref(nu), ctypes.byref(nv)))
@@ -229,7 +245,7 @@ class Surface:
     @classmethod
     def readNu(cls, path: str, stream=None) -> "Surface":
         h = _c_void()
-        _check(lib().gn_surface_from_nu(path.encode(), _c_void(stream_handle(stream)), ctypes.byref(h)))
+        _check(lib().gn_surface_from_nu(path.encode(), stream_handle(stream), ctypes.byref(h)))
         return cls(0, 0, None, None, None, None, _handle=h)
 
     def writeNu(self, path: str):
@@ -259,7 +275,7 @@ class Surface:
         torch = _torch()
         ud = to_device(u, torch.float64)
         out = torch.empty(ud.numel(), dtype=torch.int32, device="cuda")
-        _check(lib().gn_find_span(self._h, direction, ud.data_ptr(), ud.numel(), out.data_ptr(), _c_void(stream_handle(stream))))
+        _check(lib().gn_find_span(self._h, direction, ud.data_ptr(), ud.numel(), out.data_ptr(), stream_handle(stream)))
         return out
 
     def GetMatrixN(self, i: int, j: int) -> np.ndarray:
@@ -277,12 +293,12 @@ class Surface:
             ud, vd = to_device(u, torch.float64), to_device(v, torch.float64)
             n = ud.numel()
             out = out if out is not None else torch.empty((nblk, n), dtype=torch.float64, device="cuda")
-            _check(lib().gn_evaluate(self._h, ud.data_ptr(), vd.data_ptr(), n, order, out.data_ptr(), _c_void(stream_handle(stream))))
+            _check(lib().gn_evaluate(self._h, ud.data_ptr(), vd.data_ptr(), n, order, out.data_ptr(), stream_handle(stream)))
         else:
             ud, vd = to_device(u, torch.float32), to_device(v, torch.float32)
             n = ud.numel()
             out = out if out is not None else torch.empty((nblk, n), dtype=torch.float32, device="cuda")
-            _check(lib().gn_evaluate_f32(self._h, ud.data_ptr(), vd.data_ptr(), n, order, out.data_ptr(), _c_void(stream_handle(stream))))
+            _check(lib().gn_evaluate_f32(self._h, ud.data_ptr(), vd.data_ptr(), n, order, out.data_ptr(), stream_handle(stream)))
         return out
 
     EvaluateRandom = Evaluate
@@ -299,7 +315,7 @@ class Surface:
         if perm is None:
             perm = torch.empty(n, dtype=torch.int32, device="cuda")
         _check(lib().gn_evaluate_sorted_f32(self._h, ud.data_ptr(), vd.data_ptr(), n, order, out.data_ptr(),
-                                            perm.data_ptr(), _c_void(stream_handle(stream))))
+                                            perm.data_ptr(), stream_handle(stream)))
         return out, perm
 
     def EvaluateGrid(self, us, vs, order: int = 0, out=None, stream=None):
@@ -309,12 +325,12 @@ class Surface:
         nblk = (3, 9, 18)[order] if 0 <= order <= 2 else 3
         out = out if out is not None else torch.empty((nblk, ud.numel() * vd.numel()), dtype=torch.float32, device="cuda")
         _check(lib().gn_evaluate_grid_f32(self._h, ud.data_ptr(), ud.numel(), vd.data_ptr(), vd.numel(), order,
-                                          out.data_ptr(), _c_void(stream_handle(stream))))
+                                          out.data_ptr(), stream_handle(stream)))
         return out
 
     # ---- tree / seeds / inversion ----------------------------------------------------------
     def BuildTree(self, levels: int = 3, flags: int = 0, stream=None):
-        _check(lib().gn_build_tree(self._h, levels, flags, _c_void(stream_handle(stream))))
+        _check(lib().gn_build_tree(self._h, levels, flags, stream_handle(stream)))
         self.tree_levels = levels
 
     def GetTree(self):
@@ -335,7 +351,7 @@ class Surface:
 
     def BuildSeedGrid(self, resolution: int = 0, stream=None):
         """Seed grid for GN_SEED_GRID_STEP (after BuildTree; 0 picks the default resolution)."""
-        _check(lib().gn_build_seed_grid(self._h, resolution, _c_void(stream_handle(stream))))
+        _check(lib().gn_build_seed_grid(self._h, resolution, stream_handle(stream)))
 
     def GetSeedGrid(self):
         """(dims int32[3], origin float32[3], cell size, cells int32[dims] of leaf reference
@@ -361,7 +377,7 @@ class Surface:
         sv = torch.empty(n, dtype=torch.float64, device="cuda")
         _check(lib().gn_seed(self._h, mode, xd.data_ptr(), yd.data_ptr(), zd.data_ptr(), n,
                              leaf.data_ptr(), su.data_ptr(),
-                             sv.data_ptr(), _c_void(stream_handle(stream))))
+                             sv.data_ptr(), stream_handle(stream)))
         return leaf, su, sv
 
     def NewInverse(self, x, y, z, opts: Optional[InvertOpts] = None, seeds=None, out=None, stream=None,
@@ -384,13 +400,13 @@ class Surface:
             opts.seed_mode = SEED_GIVEN
         if iters is None:
             _check(lib().gn_invert(self._h, xd.data_ptr(), yd.data_ptr(), zd.data_ptr(), n, ctypes.byref(opts),
-                                   u.data_ptr(), v.data_ptr(), st.data_ptr(), _c_void(stream_handle(stream))))
+                                   u.data_ptr(), v.data_ptr(), st.data_ptr(), stream_handle(stream)))
             return u, v, st
         it32 = torch.empty(n, dtype=torch.uint8, device="cuda")
         it64 = torch.empty(n, dtype=torch.uint8, device="cuda")
         _check(lib().gn_invert_iters(self._h, xd.data_ptr(), yd.data_ptr(), zd.data_ptr(), n, ctypes.byref(opts),
                                      u.data_ptr(), v.data_ptr(), st.data_ptr(), it32.data_ptr(), it64.data_ptr(),
-                                     _c_void(stream_handle(stream))))
+                                     stream_handle(stream)))
         return u, v, st, it32, it64
 
     Invert = NewInverse
@@ -414,7 +430,7 @@ class Surface:
             v.copy_(to_device(seeds[1], torch.float64))
             opts.seed_mode = SEED_GIVEN
         _check(lib().gn_invert_noalloc(self._h, xd.data_ptr(), yd.data_ptr(), zd.data_ptr(), n, ctypes.byref(opts),
-                                       u.data_ptr(), v.data_ptr(), st.data_ptr(), _c_void(stream_handle(stream))))
+                                       u.data_ptr(), v.data_ptr(), st.data_ptr(), stream_handle(stream)))
         return u, v, st
 
     def PCurve(self, curve, samples: int, degree: int = 3, ncp: int = 16, opts: Optional[InvertOpts] = None,
@@ -429,7 +445,7 @@ class Surface:
         kn = np.zeros(ncp + degree + 1)
         dev, nf = _c_double(), _c_size()
         _check(lib().gn_pcurve(self._h, curve.handle, samples, degree, ncp, ctypes.byref(opts), cp.ctypes.data,
-                               kn.ctypes.data, ctypes.byref(dev), ctypes.byref(nf), _c_void(stream_handle(stream))))
+                               kn.ctypes.data, ctypes.byref(dev), ctypes.byref(nf), stream_handle(stream)))
         return cp.reshape(ncp, 2), kn, dev.value, nf.value
 
 
@@ -446,7 +462,7 @@ class Curve:
         k = np.ascontiguousarray(knots, dtype=np.float64)
         h = _c_void()
         _check(lib().gn_curve_create(int(degree), int(w.size), k.ctypes.data, cp.ctypes.data, w.ctypes.data,
-                                     _c_void(stream_handle(stream)), ctypes.byref(h)))
+                                     stream_handle(stream), ctypes.byref(h)))
         self._h = h
         p, n = _c_int(), _c_int()
         _check(lib().gn_curve_info(self._h, ctypes.byref(p), ctypes.byref(n)))
@@ -482,7 +498,7 @@ class Curve:
         n = td.numel()
         nblk = 3 * (order + 1) if 0 <= order <= 2 else 3
         out = out if out is not None else torch.empty((nblk, n), dtype=torch.float64, device="cuda")
-        _check(lib().gn_curve_evaluate(self._h, td.data_ptr(), n, order, out.data_ptr(), _c_void(stream_handle(stream))))
+        _check(lib().gn_curve_evaluate(self._h, td.data_ptr(), n, order, out.data_ptr(), stream_handle(stream)))
         return out
 
     def Invert(self, x, y, z, opts: Optional[InvertOpts] = None, seeds=None, out=None, stream=None):
@@ -500,7 +516,7 @@ class Curve:
             t.copy_(to_device(seeds, torch.float64))
             opts.seed_mode = SEED_GIVEN
         _check(lib().gn_curve_invert(self._h, xd.data_ptr(), yd.data_ptr(), zd.data_ptr(), n, ctypes.byref(opts),
-                                     t.data_ptr(), st.data_ptr(), _c_void(stream_handle(stream))))
+                                     t.data_ptr(), st.data_ptr(), stream_handle(stream)))
         return t, st
 
 
@@ -623,7 +639,7 @@ class Graph:
         self._h, self._keep = handle, keep
 
     def launch(self, stream=None):
-        _check(lib().gn_graph_launch(self._h, _c_void(stream_handle(stream))))
+        _check(lib().gn_graph_launch(self._h, stream_handle(stream)))
 
     def close(self):
         if self._h:
@@ -644,7 +660,7 @@ class Batch:
     def __init__(self, surfaces, stream=None):
         arr = (_c_void * len(surfaces))(*[s.handle for s in surfaces])
         h = _c_void()
-        _check(lib().gn_batch_create(arr, len(surfaces), _c_void(stream_handle(stream)), ctypes.byref(h)))
+        _check(lib().gn_batch_create(arr, len(surfaces), stream_handle(stream), ctypes.byref(h)))
         self._h = h
         self.count = len(surfaces)
         _live.add(self)
@@ -690,7 +706,7 @@ class Batch:
         opts = opts if opts is not None else default_opts()
         _check(lib().gn_batch_invert(self._h, segs.ctypes.data, len(segs), xd.data_ptr(), yd.data_ptr(), zd.data_ptr(),
                                      n, ctypes.byref(opts), u.data_ptr(), v.data_ptr(), st.data_ptr(),
-                                     _c_void(stream_handle(stream))))
+                                     stream_handle(stream)))
         return u, v, st
 
     def tune(self, segs, x, y, z, opts: Optional[InvertOpts] = None, cache_path: Optional[str] = None, out=None,
@@ -700,7 +716,7 @@ class Batch:
         opts = opts if opts is not None else default_opts()
         _check(lib().gn_batch_tune(self._h, segs.ctypes.data, len(segs), xd.data_ptr(), yd.data_ptr(), zd.data_ptr(),
                                    n, ctypes.byref(opts), u.data_ptr(), v.data_ptr(), st.data_ptr(),
-                                   cache_path.encode() if cache_path else None, _c_void(stream_handle(stream))))
+                                   cache_path.encode() if cache_path else None, stream_handle(stream)))
         return self.shape()
 
     def graph(self, segs, x, y, z, u, v, status, opts: Optional[InvertOpts] = None, stream=None) -> Graph:
@@ -711,5 +727,5 @@ class Batch:
         h = _c_void()
         _check(lib().gn_batch_graph_create(self._h, segs.ctypes.data, len(segs), x.data_ptr(), y.data_ptr(),
                                            z.data_ptr(), x.numel(), ctypes.byref(opts), u.data_ptr(), v.data_ptr(),
-                                           status.data_ptr(), _c_void(stream_handle(stream)), ctypes.byref(h)))
+                                           status.data_ptr(), stream_handle(stream), ctypes.byref(h)))
         return Graph(h, (x, y, z, u, v, status))

@@ -423,9 +423,14 @@ struct SpanCache {
     int im = 0, in = 0;  // span slots m - p, n - q
 };
 
-// Patch sources of eval_point_cached: per-lane gathers, the register-cached patch, or LDS rows
-// staged by the whole wave with the next row prefetched (wave-uniform call required).
-enum { kPatchGlobal = 0, kPatchRegs = 1, kPatchWavePipe = 2 };
+// Patch sources of eval_point_cached: per-lane gathers, the register-cached patch, LDS rows
+// staged by the whole wave with the next row prefetched (wave-uniform call required), or the lane's
+// own copy of its patch in LDS, loaded again only when its span changes.
+enum { kPatchGlobal = 0, kPatchRegs = 1, kPatchWavePipe = 2, kPatchLane = 3 };
+// 16-byte vectors between the lanes' copies (kPatchLane): odd, so that 16 lanes' reads of one vector
+// fall into different banks.
+template <int K1, int K2, typename T>
+constexpr int lane_patch_stride() { return (K1 * K2 * 4 * (int)sizeof(T) / 16) | 1; }
 
 // NEAR: the span search is find_span_near, for the batched kernels (knots in global memory, where
 // bisection's dependent loads are long) and the single-surface FP32 bulk (+2% on 1M projection
@@ -475,6 +480,17 @@ __device__ __forceinline__ void eval_point_cached(const GnSurfDev &d, const doub
                 for (int c = 0; c < K2; c++) m[c] = pr[r * K2 + c];
             },
             k1, k2, t, s, h);
+    } else if constexpr (PSRC == kPatchLane) {
+        static_assert(EXACT, "the lane's LDS patch needs exact sizes");
+        typedef float vec_t __attribute__((ext_vector_type(4)));
+        vec_t *mine = reinterpret_cast<vec_t *>(wave_lds);
+        if (moved) {
+            constexpr int nv = K1 * K2 * 4 * (int)sizeof(T) / 16;
+            const vec_t *src = reinterpret_cast<const vec_t *>(patch);
+#pragma unroll
+            for (int e = 0; e < nv; e++) mine[e] = src[e];
+        }
+        contract<K1, K2, ORDER, true, T>(reinterpret_cast<const T *>(mine), k1, k2, t, s, h);
     } else if constexpr (PSRC == kPatchWavePipe) {
         static_assert(EXACT, "LDS row staging needs exact sizes");
         (void)moved;

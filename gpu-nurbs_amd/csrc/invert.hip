@@ -1,5 +1,6 @@
 // invert.hip -- point inversion / projection entry (NewInverse + GaussNewton,
 // src/kernel/kernel.cu:151-249, 433-469): seeding, then one of
+//   small calls   k_gn_tile                    (invert_tile.hip)   seed and all iterations in one kernel
 //   plain FP64    k_gn_refill<double>          (invert_fp64.hip)   the drop-in iteration
 //   mixed         k_gn_refill<float> + k_gn_tail (invert_mixed.hip) FP32 bulk, FP64 closing steps
 //   reference     k_invert_first_hit           (invert_ref.hip)    index-order first-hit seeding
@@ -20,14 +21,16 @@ int launch_invert(const GnSurfDev &d, const GnSearchDev &sd, const GnTreeNode *t
         for (int l = 0; l < tree_levels; l++) { count += g * g; g *= 8; }
         rc = launch_gn_first_hit(d, a, tree, valid, count, st);
     } else {
-        if (o.seed_mode != GN_SEED_GIVEN) {
-            const int mode = o.seed_mode == GN_SEED_NEAREST_LEAF ? 0
-                           : o.seed_mode == GN_SEED_GREEDY_STEP  ? 2
-                           : o.seed_mode == GN_SEED_GRID_STEP    ? 3 : 1;
+        const bool given = o.seed_mode == GN_SEED_GIVEN, tile = gn_tile_takes(d, a);
+        const int mode = o.seed_mode == GN_SEED_NEAREST_LEAF ? 0
+                       : o.seed_mode == GN_SEED_GREEDY_STEP  ? 2
+                       : o.seed_mode == GN_SEED_GRID_STEP    ? 3 : 1;
+        if (!given && !(tile && mode != 0)) {
             rc = launch_seed(sd, mode, x, y, z, n, nullptr, u, v, st);
             if (rc) return rc;
         }
-        rc = o.precision == GN_MIXED ? launch_gn_mixed(d, a, st) : launch_gn_plain(d, a, st);
+        rc = tile ? launch_gn_tile(d, sd, a, given ? 0 : mode, st)
+           : o.precision == GN_MIXED ? launch_gn_mixed(d, a, st) : launch_gn_plain(d, a, st);
     }
     if (rc || !o.fallback) return rc;
     return launch_project_fallback(d, sd, a, st);

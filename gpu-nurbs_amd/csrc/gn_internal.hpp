@@ -308,6 +308,8 @@ class PoolScope {
 // ordinary kernel on st; both buffers 16-byte aligned and readable/writable to bytes rounded up
 // to 16.
 int launch_stage_copy(const void *src, void *dst, size_t bytes, hipStream_t st);
+int launch_copy_results(const double *su, const double *sv, const uint8_t *ss, size_t n, double *du,
+                        double *dv, uint8_t *ds, hipStream_t st);
 // Argument checks of gn_invert (a failing check sets the thread's error message).
 int check_invert(const gn_surface *s, const double *x, const double *y, const double *z, size_t n,
                  const gn_invert_opts &o, const double *u, const double *v, const uint8_t *status);

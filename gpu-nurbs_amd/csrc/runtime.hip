@@ -112,6 +112,32 @@ int launch_stage_copy(const void *src, void *dst, size_t bytes, hipStream_t st) 
     return GN_OK;
 }
 
+// A request's u, v (null for curves) and status into the caller's arrays, a point per lane.  Bound by the
+// launch: requests hold 64 .. 100,000 points, 17 bytes each.  A burst of 20 requests 64 .. 100,000
+// points large, submitted, answered and copied out: 690 us with three copies per request, 573 with one.
+__global__ __launch_bounds__(256) void k_copy_results(const double *__restrict__ su,
+                                                      const double *__restrict__ sv,
+                                                      const uint8_t *__restrict__ ss, size_t n,
+                                                      double *__restrict__ du,
+                                                      double *__restrict__ dv,
+                                                      uint8_t *__restrict__ ds) {
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (size_t)gridDim.x * blockDim.x) {
+        du[i] = su[i];
+        if (sv) dv[i] = sv[i];
+        ds[i] = ss[i];
+    }
+}
+
+int launch_copy_results(const double *su, const double *sv, const uint8_t *ss, size_t n, double *du,
+                        double *dv, uint8_t *ds, hipStream_t st) {
+    if (n == 0) return GN_OK;
+    const size_t blocks = (n + 255) / 256;
+    k_copy_results<<<(unsigned)(blocks < 8192 ? blocks : 8192), 256, 0, st>>>(su, sv, ss, n, du, dv, ds);
+    GN_HIP(hipGetLastError());
+    return GN_OK;
+}
+
 int blocks_per_cu(const void *kernel, int block) {
     static std::mutex mu;
     static std::unordered_map<const void *, int> cache;

@@ -579,6 +579,21 @@ int gn_server_release(gn_server *s, int64_t id) {
     return GN_OK;
 }
 
+int gn_request_copy(const gn_request_info *info, double *u, double *v, uint8_t *status,
+                    gn_stream stream) {
+    if (!info) return fail(GN_EINVAL, "null argument");
+    if (info->n == 0) return GN_OK;
+    if (!info->u || !info->status || !u || !status || (info->v && !v))
+        return fail(GN_EINVAL, "null result array");
+    hipPointerAttribute_t at{};
+    int dev = 0;
+    GN_HIP(hipGetDevice(&dev));
+    GN_HIP(hipPointerGetAttributes(&at, info->u));
+    if (at.device != dev) return fail(GN_ESTATE, "results on another device than the current one");
+    return gn::launch_copy_results(info->u, info->v, info->status, info->n, u, v, status,
+                                   (hipStream_t)stream);
+}
+
 int gn_server_stats_get(gn_server *s, gn_server_stats *stats) {
     if (!s || !stats) return fail(GN_EINVAL, "null argument");
     std::lock_guard<std::mutex> lk(s->mu);

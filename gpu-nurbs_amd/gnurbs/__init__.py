@@ -112,6 +112,7 @@ _SIGS = [
     ("gn_server_poll", _c_int, [_c_void, ctypes.c_int64, _c_void]),
     ("gn_server_wait", _c_int, [_c_void, ctypes.c_int64, _c_int, _c_void]),
     ("gn_server_release", _c_int, [_c_void, ctypes.c_int64]),
+    ("gn_request_copy", _c_int, [_c_void, _c_void, _c_void, _c_void, _c_void]),
     ("gn_server_stats_get", _c_int, [_c_void, _c_void]),
     ("gn_server_destroy", _c_int, [_c_void]),
     ("gn_now_ns", ctypes.c_int64, []),
@@ -606,6 +607,14 @@ class Server:
         for curves, as device tensors."""
         torch = _torch()
         n = info.n
+        u = torch.empty(n, dtype=torch.float64, device="cuda")
+        v = torch.empty(n, dtype=torch.float64, device="cuda") if info.v else None
+        st = torch.empty(n, dtype=torch.uint8, device="cuda")
+        rc = lib().gn_request_copy(ctypes.byref(info), u.data_ptr(), v.data_ptr() if info.v else None, st.data_ptr(),
+                                   stream_handle())
+        if rc != GN_ESTATE:
+            _check(rc)
+            return u, v, st
         u = torch.as_tensor(_DeviceView(info.u, n, "<f8"), device="cuda").clone()
         v = torch.as_tensor(_DeviceView(info.v, n, "<f8"), device="cuda").clone() if info.v else None
         st = torch.as_tensor(_DeviceView(info.status, n, "|u1"), device="cuda").clone()

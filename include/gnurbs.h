@@ -369,6 +369,11 @@ int gn_server_poll(gn_server *s, int64_t id, gn_request_info *info);
 int gn_server_wait(gn_server *s, int64_t id, int timeout_ms, gn_request_info *info);
 /* Frees a finished request's results (GN_ESTATE while it is still queued or running). */
 int gn_server_release(gn_server *s, int64_t id);
+/* Copies a finished, unreleased request's results into device arrays of info->n elements (v may be
+ * NULL where info->v is) in the order of stream.  GN_ESTATE if they are on another device than the
+ * current one. */
+int gn_request_copy(const gn_request_info *info, double *u, double *v, uint8_t *status,
+                    gn_stream stream);
 int gn_server_stats_get(gn_server *s, gn_server_stats *stats);
 /* Finishes the steps in flight, fails the requests not yet launched, frees the arena. */
 int gn_server_destroy(gn_server *s);

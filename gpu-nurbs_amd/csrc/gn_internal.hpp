@@ -243,7 +243,7 @@ struct GroupRange {
 };
 std::vector<GroupRange> group_ranges(const GnTile *tiles, size_t ntiles, const std::vector<int> &cls);
 // Points per tile for a launch of `points` points: about two tiles per resident wave, between 64
-// and cap (a tile is the unit a wave claims; too large a tile leaves waves idle).
+// and cap (a larger tile shortens the list, and leaves more workgroups without points at its end).
 int class_tile(size_t points, int waves, int cap);
 // Side streams and fork/join events for running independent launches concurrently.  A set is
 // used by one caller at a time (the batched entry points share one per device under a lock; a
@@ -257,8 +257,7 @@ int side_streams_create(SideStreams *ss);
 // Creates the device's shared side-stream set (call before a graph capture).
 int batch_prepare();
 void side_streams_destroy(SideStreams *ss);
-// Per group range: seeds (unless GN_SEED_GIVEN), then one persistent launch per precision
-// phase.  The groups run concurrently on the side streams (forked from and joined back into st);
+// Per group range one launch, after one of nearest-leaf seeds where they are asked for.  The groups run concurrently on the side streams (forked from and joined back into st);
 // `beside`, if given, enqueues further work on st that runs alongside them.  With side ==
 // nullptr the device's shared set is used.  group_done, if given, receives (group, event) for
 // every group that ran on a side stream: the event completes when that group's work has (it is
@@ -270,7 +269,7 @@ int launch_batch_invert(const GnBatchObj *objs, const GnTile *tiles,
                         const SideStreams *side = nullptr,
                         const std::function<int(hipStream_t)> &beside = {},
                         std::vector<std::pair<int, hipEvent_t>> *group_done = nullptr);
-// resident waves of one persistent batch launch (sizes tiles for short serving steps)
+// resident waves of one batch launch (sizes tiles)
 int batch_waves(int bpc_cap);
 // tiles of curve objects (obj indexes `curves`); max_samples: largest seed sample count
 int launch_curve_batch(const GnCurveDev *curves, const GnTile *tiles, int ntiles, const GnReq *reqs,

@@ -416,7 +416,7 @@ inline void refill_shape(const void *kernel, size_t n, unsigned &grid, int &slic
 // launchers, one translation unit each (invert_fp64.hip, invert_mixed.hip, invert_ref.hip,
 // project.hip)
 int launch_gn_plain(const GnSurfDev &d, const InvArgs &a, hipStream_t st);
-// one launch from seed to result for small calls (invert_tile.hip)
+// one launch from seed to result (invert_tile.hip)
 bool gn_tile_takes(const GnSurfDev &d, const InvArgs &a);
 int launch_gn_tile(const GnSurfDev &d, const GnSearchDev &sd, const InvArgs &a, int seed,
                    hipStream_t st);

@@ -1,13 +1,8 @@
 // invert_tile.hip -- inversion of calls of up to a few points per lane of the chip: the seed, the FP32
 // bulk and the FP64 iterations of a point in one kernel.
-#include "gn_search.hpp"
-#include "invert_common.hpp"
+#include "invert_tile.hpp"
 
 namespace gn {
-
-// Levels of the seed quadtree whose boxes a wave stages (with the root 341 boxes, 8 KB): what the
-// smallest patches' LDS holds.
-constexpr int kTileSeedLevels = 4;
 
 // Every lane keeps one point from its seed to its result; a wave is a workgroup, so a call of n
 // points is n / 64 waves on as many CUs as there are.  What bounds a small call is the latency of
@@ -21,13 +16,11 @@ constexpr int kTileSeedLevels = 4;
 // bicubic 26.5 -> 14.3 us, 32 x 32 72.6 -> 46.2, degree (4,4) 94 -> 60; mixed 31 -> 11, 47.5 -> 20.8
 // and 57 -> 28.  Of the 46 us, 22 iterations of the slowest lane are 1.6 us each.
 
-// seed: 0 the parameters in a.u, a.v; 1 the greedy descent's leaf, 2 with its step; 3 the seed grid's
-// leaf with its step.
+// seed: 0 the parameters in a.u, a.v, else as tile_seed.
 template <int K1, int K2, bool MIXED, bool NEWTON32, bool NEWTON64>
 __global__ __launch_bounds__(64, 1) void k_gn_tile(GnSurfDev d_in, GnSearchDev sd, InvArgs a,
                                                    int seed) {
-    constexpr int kStride = lane_patch_stride<K1, K2, double>();
-    __shared__ float4 patches[64 * kStride];
+    __shared__ float4 patches[tile_patch_vecs<K1, K2, MIXED>()];
     extern __shared__ double sk[];
     const size_t i = (size_t)blockIdx.x * 64 + threadIdx.x;
     const bool valid = i < a.n;
@@ -41,75 +34,19 @@ __global__ __launch_bounds__(64, 1) void k_gn_tile(GnSurfDev d_in, GnSearchDev s
             cv = a.v[i];
         }
     }
-    int ll = 0;
-    if (seed == 1 || seed == 2) {  // the boxes of levels 0..ll, where the patches go afterwards
-        static_assert((((1 << (2 * (kTileSeedLevels + 1))) - 1) / 3) * 24 <= sizeof(patches), "");
-        ll = sd.depth < kTileSeedLevels ? sd.depth : kTileSeedLevels;
-        const float2 *src = reinterpret_cast<const float2 *>(sd.box32);
-        float2 *dst = reinterpret_cast<float2 *>(patches);
-        const int nf2 = (int)qoff(ll + 1) * 3;
-#pragma unroll 8
-        for (int e = threadIdx.x; e < nf2; e += 64) dst[e] = src[e];
-    }
+    const int ll = tile_stage_boxes(sd, seed, patches);
     const GnSurfDev d = stage_knots_lds(d_in, sk);
-    if (seed != 0 && valid) {
-        if (seed == 3) {
-            const uint32_t c = sd.grid_wide ? grid_leaf<true>(sd, P) : grid_leaf<false>(sd, P);
-            step_seed(sd, c, sd.rec[(size_t)c * kRecVec], P, cu, cv);
-        } else {
-            float4 cq;
-            const uint32_t c = greedy_leaf(sd, P, reinterpret_cast<const float *>(patches) + 6, ll,
-                                           &cq, seed == 1);
-            if (seed == 2) {
-                step_seed(sd, c, cq, P, cu, cv);
-            } else {
-                cu = sd.seed_uv[c * 2 + 0];
-                cv = sd.seed_uv[c * 2 + 1];
-            }
-        }
-    }
+    if (seed != 0 && valid) tile_seed(sd, seed, patches, ll, P, cu, cv);
     __syncthreads();  // every lane has left the boxes
-    const double *ku = sk, *kv = sk + d.nu + d.p + 1;
-    const Domain dom = domain_of(d);
-    int lim = a.o.max_iter;
-    if constexpr (MIXED) {
-        const double su = cu, sv = cv;
-        SpanCache sc;
-        int it = 0, st = valid && a.o.fp32_iters > 0 ? kStepContinue : GN_PT_MAXITER;
-        while (st == kStepContinue) {
-            st = gn_step<K1, K2, true, float, NEWTON32, kPatchLane, false, true>(
-                d, ku, kv, (float)P[0], (float)P[1], (float)P[2], cu, cv, 0.0, a.o.tol_step32, 0.0,
-                a.o.clamp, dom, sc, nullptr,
-                patches + threadIdx.x * lane_patch_stride<K1, K2, float>());
-            if (st == kStepContinue || st == GN_PT_CONVERGED) it++;
-            if (st == kStepContinue && it >= a.o.fp32_iters) st = GN_PT_MAXITER;
-        }
-        if (valid && a.it32) a.it32[i] = sat8(it);
-        if (st == GN_PT_SINGULAR || st == GN_PT_NONFINITE) {
-            cu = su;
-            cv = sv;
-        } else {
-            lim = a.o.fp64_tail;
-        }
-        __syncthreads();
-    } else {
-        if (valid && a.it32) a.it32[i] = 0;
-    }
-    const double tq = NEWTON64 ? a.o.tol_quad : 0.0;
-    SpanCache sc;
-    int it = 0, st = valid && lim > 0 ? kStepContinue : GN_PT_MAXITER;
-    while (st == kStepContinue) {
-        st = gn_step<K1, K2, true, double, NEWTON64, kPatchLane, false, true>(
-            d, ku, kv, P[0], P[1], P[2], cu, cv, a.o.tol_dist, a.o.tol_step, tq, a.o.clamp, dom, sc,
-            nullptr, patches + threadIdx.x * kStride);
-        if (st == kStepContinue || st == GN_PT_CONVERGED) it++;
-        if (st == kStepContinue && it >= lim) st = GN_PT_MAXITER;
-    }
+    int it32, it64;
+    const int st = tile_iterate<K1, K2, true, MIXED, NEWTON32, NEWTON64>(
+        d, sk, sk + d.nu + d.p + 1, domain_of(d), a.o, P, valid, patches, cu, cv, it32, it64);
     if (!valid) return;
     a.u[i] = cu;
     a.v[i] = cv;
     a.status[i] = (uint8_t)st;
-    if (a.it64) a.it64[i] = sat8(it);
+    if (a.it32) a.it32[i] = sat8(it32);
+    if (a.it64) a.it64[i] = sat8(it64);
 }
 
 struct TileLaunch {
@@ -137,25 +74,24 @@ struct TileLaunch {
     }
 };
 
-// Waves of this kernel that a CU's 160 KB of LDS hold (registers would allow four to eight).
-static int tile_waves_per_cu(const GnSurfDev &d) {
-    const size_t vec = (size_t)((d.p + 1) * (d.q + 1) * 2) | 1;
-    return (int)((160 * 1024) / (vec * 16 * 64 + sizeof(double) * (2 * (d.nu + d.nv) + 2)));
-}
-
-// Whether the call runs faster here than as seeds plus persistent kernels.  A round is as many
-// points as the chip's LDS holds patches for: 65,536 for bicubic FP64, 114,688 biquadratic, 32,768
-// of degree (5,5).  Within one round this kernel always wins (FP64: (3,3) 46 against 72 us at 4,096
-// points, 63 against 77 at 65,536; (5,5) 102 against 171 at 16,000; mixed: (3,3) 21 against 47 and
-// 26 against 50).  Past it the persistent kernels refill lanes whose points have stopped, this one
-// starts over: FP64 (3,3) 87 against 105 us at 80,000 but 114 against 105 at 131,072, (2,2) 112
-// against 150 at 320,000, (5,5) 201 against 146 at 65,000; mixed (3,3) 44 against 57 at 131,072 and
-// 76 against 72 at 250,001, (2,2) 50 against 70 at 320,000, (5,5) 78 against 73 at 65,000.
+// Whether the call runs faster here than as seeds plus persistent kernels, which refill lanes whose
+// points have stopped where this kernel starts a new wave and waits for its slowest lane.
+// Mixed precision: up to 31,250 points per CU times the patch entries, more for 3 x 3.  Here against
+// there, us: (3,3) 30 / 56 at 70,000 points, 121 / 121 at 600,000, 191 / 167 at 1,000,000; (2,3) 119 /
+// 123 at 600,000, 155 / 144 at 800,000; (4,4) 118 / 123 at 300,000, 152 / 146 at 400,000; (5,5) 114 /
+// 130 at 200,000, 157 / 150 at 300,000; (2,2) 99 / 134 at 1,000,000.
+// FP64: by rounds, as many points as the chip's LDS holds patches for (65,536 bicubic, 114,688
+// biquadratic, 32,768 of degree (5,5)).  One always wins: (3,3) 46 / 72 at 4,096, 63 / 77 at 65,536;
+// (5,5) 102 / 171 at 16,000.  Past it (3,3) 87 / 105 at 80,000, 114 / 105 at 131,072; (2,2) 112 / 150
+// at 320,000; (5,5) 201 / 146 at 65,000.
 bool gn_tile_takes(const GnSurfDev &d, const InvArgs &a) {
     if (!knots_fit_lds(d) || d.p < 2 || d.p > 5 || d.q < 2 || d.q > 5) return false;
-    const int w = tile_waves_per_cu(d);
-    const int halves = w >= 6 ? 6 : a.o.precision != GN_MIXED ? (w >= 4 ? 3 : 2) : w >= 3 ? 4 : 3;
-    return a.n <= (size_t)cu_count() * 32 * w * halves;
+    const size_t entries = (size_t)((d.p + 1) * (d.q + 1)), cus = (size_t)cu_count();
+    if (a.o.precision == GN_MIXED)
+        return entries <= 9 ? a.n < ((size_t)1 << 31) : a.n * entries <= 31250 * cus;
+    const size_t lds = ((entries * 2) | 1) * 16 * 64 + sizeof(double) * (2 * (d.nu + d.nv) + 2);
+    const size_t w = 160 * 1024 / lds;  // waves per CU
+    return a.n <= cus * 32 * w * (w >= 6 ? 6 : w >= 4 ? 3 : 2);
 }
 
 int launch_gn_tile(const GnSurfDev &d, const GnSearchDev &sd, const InvArgs &a, int seed,

@@ -263,12 +263,12 @@ typedef struct gn_graph gn_graph; /* an instantiated hipGraph of one batched inv
 int gn_batch_create(gn_surface *const *surfaces, int count, gn_stream stream, gn_batch **out);
 int gn_batch_destroy(gn_batch *b);
 size_t gn_batch_device_bytes(const gn_batch *b);
-/* Tile shape: points per tile (work unit claimed by one wave) and a cap on resident workgroups
- * per CU (0 = occupancy limit). */
+/* Tile shape: points per tile at most (entries of the work list; a wave takes 64 of a tile's points)
+ * and a cap on resident workgroups of 256 lanes per CU (0 = occupancy limit). */
 int gn_batch_set_shape(gn_batch *b, int tile_points, int blocks_per_cu);
 int gn_batch_get_shape(const gn_batch *b, int *tile_points, int *blocks_per_cu);
 /* Inverts the points of all segments (device arrays x, y, z, u, v, status of length n) with one
- * persistent launch per precision phase; seeds: GN_SEED_GREEDY_LEAF, GN_SEED_NEAREST_LEAF,
+ * launch per group of degree classes; seeds: GN_SEED_GREEDY_LEAF, GN_SEED_NEAREST_LEAF,
  * GN_SEED_GREEDY_STEP, GN_SEED_GRID_STEP (each point on its own surface's tree or grid) or
  * GN_SEED_GIVEN. */
 int gn_batch_invert(gn_batch *b, const gn_segment *segs, int nseg, const double *x,

@@ -232,8 +232,17 @@ static int launch_ranges(const GnBatchObj *objs, const GnTile *tiles,
     // may then synchronise st alone (or free buffers in its order) before it reuses what the
     // kernels already enqueued still read or write
     int k = 0, rc = GN_OK;
-    for (const GroupRange &gr : ranges) {
+    // the group of the largest patches, whose points take longest, first: on st itself, without the
+    // wait for the fork, where nothing else has to run there
+    const bool own = !beside && !group_done;
+    for (auto it = ranges.rbegin(); it != ranges.rend(); ++it) {
+        const GroupRange &gr = *it;
         if (gr.points == 0) continue;
+        if (own && it == ranges.rbegin()) {
+            rc = run_range(objs, tiles, gr, reqs, o, bpc_cap, st);
+            if (rc) break;
+            continue;
+        }
         const hipError_t e = hipStreamWaitEvent(ss.s[k], ss.fork, 0);
         if (e != hipSuccess) {
             rc = hip_fail(e, "hipStreamWaitEvent(fork)");

@@ -2,7 +2,7 @@
 // src/kernel/kernel.cu:151-249, 433-469): seeding, then one of
 //   small calls   k_gn_tile                    (invert_tile.hip)   seed and all iterations in one kernel
 //   plain FP64    k_gn_refill<double>          (invert_fp64.hip)   the drop-in iteration
-//   mixed         k_gn_refill<float> + k_gn_tail (invert_mixed.hip) FP32 bulk, FP64 closing steps
+//   mixed         k_gn_refill<float> + k_close_first + k_gn_refill<kCloseList> (invert_mixed.hip)
 //   reference     k_invert_first_hit           (invert_ref.hip)    index-order first-hit seeding
 #include "invert_common.hpp"
 

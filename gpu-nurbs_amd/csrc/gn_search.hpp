@@ -128,7 +128,10 @@ __device__ inline uint32_t greedy_leaf(const GnSearchDev &sd, const double P[3],
                                        const float *lds = nullptr, int lds_levels = 0,
                                        float4 *cbest = nullptr, bool refine = true) {
     const int D = sd.depth;
-    if (D == 0) return 0;
+    if (D == 0) {
+        if (cbest) *cbest = sd.rec[0];
+        return 0;
+    }
     const float p[3] = {(float)P[0], (float)P[1], (float)P[2]};
     uint32_t c = 0;
     int l = 0;

@@ -14,11 +14,12 @@ LARGE = 700_001  # beyond the rule for every degree (at most three rounds of 7 w
 MIXED = dict(precision=G.GN_MIXED, fp32_iters=6, fp64_tail=3, tol_step32=3e-5, tol_step=1e-10, tol_quad=1e-10)
 
 
-def _surface(p, q, nu, nv):
+def _surface(p, q, nu, nv, levels=3):
     sd = synth.surface_G(nu, nv, p, q, seed=17, jitter=0.3)
     g = G.Surface(sd.p, sd.q, sd.ku, sd.kv, sd.cp, sd.w)
-    g.BuildTree(3)
-    g.BuildSeedGrid(0)
+    g.BuildTree(levels)
+    if levels > 1:
+        g.BuildSeedGrid(0)
     return g
 
 
@@ -82,3 +83,16 @@ def test_sizes_around_the_rule(p, q, n):
     P = _points(g, n, 6)
     _same(g, P, G.default_opts(newton=2), n, False)
     _same(g, P, G.default_opts(seed_mode=G.SEED_GRID_STEP, newton=3, **MIXED), n, False)
+
+
+def test_a_tree_of_one_leaf():
+    """The stepped seed of the only leaf starts from that leaf's centre, as gn_seed's does."""
+    g = _surface(3, 3, 8, 8, levels=1)
+    P = _points(g, 300, 4)
+    _, su, sv = g.Seed(*P, exact="step")
+    given = [su.clone(), sv.clone(), torch.empty(300, dtype=torch.uint8, device="cuda")]
+    g.NewInverse(*P, G.default_opts(seed_mode=G.SEED_GIVEN, newton=2), out=given)
+    got = g.NewInverse(*P, G.default_opts(seed_mode=G.SEED_GREEDY_STEP, newton=2))
+    for a, b in zip(got, given):
+        assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+    _same(g, P, G.default_opts(seed_mode=G.SEED_GREEDY_STEP, newton=2), 300, False)

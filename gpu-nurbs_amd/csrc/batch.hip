@@ -10,6 +10,8 @@
 // group alone, so a launch has the registers and LDS of its group -- one kernel holding every class
 // would be sized by the largest.  A workgroup is one wave: 64 points of one tile, seeded and
 // iterated to the end on their lanes (invert_tile.hpp), so the class dispatch is workgroup-uniform.
+// Where many rounds of such waves would wait for their slowest lanes, the group takes the persistent
+// kernels of batch_refill.hip (batch_takes_refill).
 // Point arrays are addressed through a request table (GnReq): a tile names its request, so one
 // launch serves the points of many independent requests (the serving loop) or of one call (a
 // one-entry table).
@@ -17,30 +19,9 @@
 #include <mutex>
 
 #include "invert_tile.hpp"
+#include "path_rules.hpp"
 
 namespace gn {
-
-// Nearest-leaf seeds of every point of the tiles into its request's u, v (the exact search walks the
-// tree; the other seeds are found in the kernel that iterates).  Workgroup b takes the points
-// (b % per_tile) * kSeedBlock .. + kSeedBlock - 1 of tile b / per_tile, one point per lane.
-constexpr int kSeedBlock = 256;
-__global__ __launch_bounds__(kSeedBlock) void k_batch_seed(const GnBatchObj *__restrict__ objs,
-                                                           const GnTile *__restrict__ tiles,
-                                                           long long nblocks, int per_tile,
-                                                           const GnReq *__restrict__ reqs) {
-    for (long long b = blockIdx.x; b < nblocks; b += gridDim.x) {  // workgroup-uniform
-        const GnTile tl = tiles[b / per_tile];
-        const GnSearchDev sd = global_view(objs[tl.obj].sd);
-        const int j = (int)(b % per_tile) * kSeedBlock + threadIdx.x;
-        if (j >= tl.count) continue;
-        const GnReq R = global_view(reqs[tl.req]);
-        const int64_t i = tl.start + j;
-        const double P[3] = {R.x[i], R.y[i], R.z[i]};
-        const uint32_t c = nearest_leaf(sd, P);
-        R.u[i] = sd.seed_uv[c * 2 + 0];
-        R.v[i] = sd.seed_uv[c * 2 + 1];
-    }
-}
 
 struct BatchTileArgs {
     const GnBatchObj *objs;
@@ -202,17 +183,18 @@ SideStreams g_side[64];  // per device, created on first use
 
 static int run_range(const GnBatchObj *objs, const GnTile *tiles, const GroupRange &gr,
                      const GnReq *reqs, const gn_invert_opts &o, int bpc_cap, hipStream_t st) {
-    const int ntiles = gr.t1 - gr.t0, longest = std::max(gr.max_count, 1);
-    if (o.seed_mode == GN_SEED_NEAREST_LEAF) {
-        const int per_tile = (longest + kSeedBlock - 1) / kSeedBlock;
-        const long long nb = (long long)ntiles * per_tile;
-        const unsigned grid = (unsigned)(nb < (1 << 20) ? nb : (1 << 20));
-        k_batch_seed<<<grid, kSeedBlock, 0, st>>>(objs, tiles + gr.t0, nb, per_tile, reqs);
-        GN_HIP(hipGetLastError());
+    const PathOpts limits{o.precision == GN_MIXED, (o.newton & GN_NEWTON_FP64) != 0, o.max_iter,
+                          o.fp32_iters, o.fp64_tail};
+    const bool refill = batch_takes_refill(gr.grp, gr.points, limits, (size_t)cu_count());
+    if (o.seed_mode != GN_SEED_GIVEN && (refill || o.seed_mode == GN_SEED_NEAREST_LEAF)) {
+        const int rc = launch_batch_seed(objs, tiles, gr, reqs, o.seed_mode, st);
+        if (rc) return rc;
     }
+    if (refill) return launch_batch_refill(objs, tiles, gr, reqs, o, bpc_cap, st);
     const int seed = o.seed_mode == GN_SEED_GREEDY_LEAF ? 1 : o.seed_mode == GN_SEED_GREEDY_STEP ? 2
                    : o.seed_mode == GN_SEED_GRID_STEP ? 3 : 0;
-    const BatchTileArgs a{objs, tiles + gr.t0, reqs, (longest + 63) / 64, seed, o};
+    const int ntiles = gr.t1 - gr.t0;
+    const BatchTileArgs a{objs, tiles + gr.t0, reqs, (std::max(gr.max_count, 1) + 63) / 64, seed, o};
     return gr.grp == 0 ? launch_group<0>(a, ntiles, bpc_cap, st)
          : gr.grp == 1 ? launch_group<1>(a, ntiles, bpc_cap, st)
                        : launch_group<2>(a, ntiles, bpc_cap, st);

@@ -257,7 +257,9 @@ int side_streams_create(SideStreams *ss);
 // Creates the device's shared side-stream set (call before a graph capture).
 int batch_prepare();
 void side_streams_destroy(SideStreams *ss);
-// Per group range one launch, after one of nearest-leaf seeds where they are asked for.  The groups run concurrently on the side streams (forked from and joined back into st);
+// Per group range one launch (batch.hip), or the persistent launches of batch_refill.hip where their
+// rule says so (path_rules.hpp); a seed launch before the latter, and for nearest-leaf seeds.  The
+// groups run concurrently on the side streams (forked from and joined back into st);
 // `beside`, if given, enqueues further work on st that runs alongside them.  With side ==
 // nullptr the device's shared set is used.  group_done, if given, receives (group, event) for
 // every group that ran on a side stream: the event completes when that group's work has (it is
@@ -269,6 +271,12 @@ int launch_batch_invert(const GnBatchObj *objs, const GnTile *tiles,
                         const SideStreams *side = nullptr,
                         const std::function<int(hipStream_t)> &beside = {},
                         std::vector<std::pair<int, hipEvent_t>> *group_done = nullptr);
+// Seeds of a group range's points into their requests' u, v, and the range's persistent launches from
+// them (batch_refill.hip).
+int launch_batch_seed(const GnBatchObj *objs, const GnTile *tiles, const GroupRange &gr,
+                      const GnReq *reqs, int seed_mode, hipStream_t st);
+int launch_batch_refill(const GnBatchObj *objs, const GnTile *tiles, const GroupRange &gr,
+                        const GnReq *reqs, const gn_invert_opts &o, int bpc_cap, hipStream_t st);
 // resident waves of one batch launch (sizes tiles)
 int batch_waves(int bpc_cap);
 // tiles of curve objects (obj indexes `curves`); max_samples: largest seed sample count

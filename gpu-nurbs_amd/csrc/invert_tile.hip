@@ -1,6 +1,7 @@
 // invert_tile.hip -- inversion of calls of up to a few points per lane of the chip: the seed, the FP32
 // bulk and the FP64 iterations of a point in one kernel.
 #include "invert_tile.hpp"
+#include "path_rules.hpp"
 
 namespace gn {
 
@@ -74,24 +75,10 @@ struct TileLaunch {
     }
 };
 
-// Whether the call runs faster here than as seeds plus persistent kernels, which refill lanes whose
-// points have stopped where this kernel starts a new wave and waits for its slowest lane.
-// Mixed precision: up to 31,250 points per CU times the patch entries, more for 3 x 3.  Here against
-// there, us: (3,3) 30 / 56 at 70,000 points, 121 / 121 at 600,000, 191 / 167 at 1,000,000; (2,3) 119 /
-// 123 at 600,000, 155 / 144 at 800,000; (4,4) 118 / 123 at 300,000, 152 / 146 at 400,000; (5,5) 114 /
-// 130 at 200,000, 157 / 150 at 300,000; (2,2) 99 / 134 at 1,000,000.
-// FP64: by rounds, as many points as the chip's LDS holds patches for (65,536 bicubic, 114,688
-// biquadratic, 32,768 of degree (5,5)).  One always wins: (3,3) 46 / 72 at 4,096, 63 / 77 at 65,536;
-// (5,5) 102 / 171 at 16,000.  Past it (3,3) 87 / 105 at 80,000, 114 / 105 at 131,072; (2,2) 112 / 150
-// at 320,000; (5,5) 201 / 146 at 65,000.
 bool gn_tile_takes(const GnSurfDev &d, const InvArgs &a) {
-    if (!knots_fit_lds(d) || d.p < 2 || d.p > 5 || d.q < 2 || d.q > 5) return false;
-    const size_t entries = (size_t)((d.p + 1) * (d.q + 1)), cus = (size_t)cu_count();
-    if (a.o.precision == GN_MIXED)
-        return entries <= 9 ? a.n < ((size_t)1 << 31) : a.n * entries <= 31250 * cus;
-    const size_t lds = ((entries * 2) | 1) * 16 * 64 + sizeof(double) * (2 * (d.nu + d.nv) + 2);
-    const size_t w = 160 * 1024 / lds;  // waves per CU
-    return a.n <= cus * 32 * w * (w >= 6 ? 6 : w >= 4 ? 3 : 2);
+    const PathOpts o{a.o.precision == GN_MIXED, (a.o.newton & GN_NEWTON_FP64) != 0, a.o.max_iter,
+                     a.o.fp32_iters, a.o.fp64_tail};
+    return call_takes_tile(d.p, d.q, (size_t)(d.nu + d.p + 1 + d.nv + d.q + 1), a.n, o, (size_t)cu_count());
 }
 
 int launch_gn_tile(const GnSurfDev &d, const GnSearchDev &sd, const InvArgs &a, int seed,

@@ -16,6 +16,39 @@ inline size_t chain_limit(const PathOpts &o) {
     return o.mixed ? (size_t)o.fp32_iters + 3 * (size_t)o.fp64_tail : (size_t)o.max_iter;
 }
 
+// Single-surface calls of exact degrees (2..5) with their knots in LDS: whether `n` points go from seed to
+// result in one kernel (k_gn_tile), or to seeds and the persistent kernels, which refill lanes whose
+// points have stopped where that kernel starts a new wave and waits for its slowest lane.  knots: of both
+// directions.  All ratios are persistent / tile, without / with 2% of the points anywhere.
+// Mixed: points times patch entries times chain limit up to 120 M on 256 CUs.  6 FP32 and 3 FP64 steps
+// (15): (3,3) 1.26 / 1.15 at 262,144 points, 1.10 / 0.96 at 500,000, 0.91 / 0.77 at 1,000,000; (5,5) 1.25 / 1.09 at
+// 131,072, 1.08 / 0.84 at 262,144.  20 and 3 (29): (3,3) 1.21 / 0.97 at 262,144, 1.03 / 0.73 at 500,000; (5,5) 1.55 /
+// 1.28 at 65,536, 1.37 / 0.86 at 131,072.  6 and 12 (42): (3,3) 1.07 / 1.17 at 131,072, 1.03 / 0.86 at 262,144.  30
+// and 40 (150): (3,3) 1.08 / 0.96 at 65,536, 0.84 / 0.96 at 131,072; (5,5) 1.24 / 1.25 at 32,768, 1.04 / 0.86 at
+// 65,536: whatever the limit, 98,304 bicubic points win or lose little.  A patch of 9 entries counts as 5:
+// (2,2) 1.26 / 0.98 at 500,000 points for 29; for 15 it wins nearly always, 1.28 / 1.12 at 1,000,000, 1.04 / 0.92 at
+// 4,000,000, 1.16 / 1.11 at 16,000,000.  Without Newton steps in FP64 the persistent closing pass is the
+// slower one, and the limit counts half: 20 and 3, (3,3) 1.47 / 1.38 at 262,144, 1.05 / 0.93 at 500,000.
+// FP64: by rounds, as many points as the chip's LDS holds patches for (65,536 bicubic, 114,688 biquadratic,
+// 32,768 of degree (5,5)); 20 Gauss-Newton steps: one round always wins, (3,3) 1.19 / 1.17 at 65,536, 0.91 / 0.86
+// at 131,072; (2,2) 1.29 / 1.27 at 262,144; (5,5) 1.13 / 1.05 at 32,768, 0.61 / 0.57 at 65,536.  Newton steps end
+// most points early, half as many: (3,3) 1.07 / 1.11 at 32,768, 0.92 / 0.90 at 65,536; (2,2) 1.08 / 1.11 at 131,072,
+// 0.92 / 0.86 at 262,144.  More than 20 steps, a third: 50 Newton steps (3,3) 0.95 / 1.02 at 32,768, 0.81 / 0.79 at
+// 65,536; 100 Gauss-Newton steps (2,2) 1.09 / 1.13 at 131,072, 0.78 / 0.74 at 262,144.
+inline bool call_takes_tile(int p, int q, size_t knots, size_t n, const PathOpts &o, size_t cus) {
+    if (knots > 1024 || p < 2 || p > 5 || q < 2 || q > 5) return false;
+    const size_t entries = (size_t)((p + 1) * (q + 1)), limit = chain_limit(o);
+    if (o.mixed)
+        return n * entries <= 6144 * cus ||
+               (n < ((size_t)1 << 31) &&
+                ((entries <= 9 && limit <= 16) ||
+                 n * (entries <= 9 ? 5 : entries) * limit <= 468750 * cus * (o.newton64 ? 1 : 2)));
+    // a wave's LDS: the lanes' patches; knots and reciprocal span lengths, two of them short of the knots
+    const size_t lds = ((entries * 2) | 1) * 16 * 64 + sizeof(double) * 2 * (knots - p - q - 1);
+    const size_t w = 160 * 1024 / lds, most = cus * 32 * w * (w >= 6 ? 6 : w >= 4 ? 3 : 2);
+    return n <= (limit > 20 ? most / 3 : o.newton64 ? most / 2 : most);
+}
+
 // Batched calls: whether a class group's `points` go to the persistent kernels (batch_refill.hip), whose
 // lanes take another point when theirs has stopped, and not to k_batch_tile, whose waves end with their
 // slowest lane.  k_batch_tile needs one launch and keeps the lanes' patches at hand, and wins wherever

@@ -7,6 +7,7 @@ import subprocess
 import pytest
 
 import test_gpu_batch_refill as batch_refill
+import test_gpu_persistent_calls as persistent
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -15,12 +16,13 @@ DRIVER = r"""
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-// batch GRP POINTS, then MIXED NEWTON64 MAX_ITER FP32_ITERS FP64_TAIL: 1 if persistent
+// batch GRP POINTS | call P Q KNOTS POINTS, then MIXED NEWTON64 MAX_ITER FP32_ITERS FP64_TAIL: 1 if persistent
 int main(int argc, char **argv) {
     auto n = [&](int k) { return (size_t)atoll(argv[k]); };
     const int at = argc - 5;
     const gn::PathOpts o{n(at) != 0, n(at + 1) != 0, (int)n(at + 2), (int)n(at + 3), (int)n(at + 4)};
     if (!strcmp(argv[1], "batch")) printf("%d", (int)gn::batch_takes_refill((int)n(2), n(3), o, 256));
+    else printf("%d", (int)!gn::call_takes_tile((int)n(2), (int)n(3), n(4), n(5), o, 256));
     return 0;
 }
 """
@@ -58,3 +60,30 @@ def test_batch_rule(rule):
             assert rule("batch", grp, 8 * half, mixed=mixed, newton64=True, max_iter=100, fp32_iters=30, fp64_tail=40)
     assert not rule("batch", 0, 1 << 24, max_iter=20) and rule("batch", 0, 1 << 24, max_iter=21)
     assert not rule("batch", 0, 1 << 24, mixed=True, fp32_iters=6, fp64_tail=3)
+
+
+def _call(rule, p, q, n, opts, newton64=True):
+    knots = 20 + p + 1 + 23 + q + 1
+    return rule("call", p, q, knots, n, mixed=True, newton64=newton64, fp32_iters=opts.get("fp32_iters", 20),
+                fp64_tail=opts.get("fp64_tail", 3))
+
+
+def test_calls_of_the_persistent_tests_are_persistent(rule):
+    for p, q, opts, n in persistent.BITS:
+        assert _call(rule, p, q, n, opts) and not _call(rule, p, q, persistent.SMALL, opts), (p, q, n)
+    assert all(_call(rule, 3, 3, n, persistent.SHORT) for n in persistent.NOALLOC)
+    assert _call(rule, 3, 3, persistent.STREAMS, persistent.DEFAULT)
+    assert _call(rule, 2, 2, persistent.SLOW, persistent.LONG)
+
+
+def test_call_rule(rule):
+    """Every class reaches both sides, in both precisions; other degrees and long knot vectors never the tile."""
+    for p in range(2, 6):
+        for q in range(2, 6):
+            for mixed in (False, True):
+                assert not rule("call", p, q, 60, 4096, mixed=mixed) and rule("call", p, q, 60, 1 << 23, mixed=mixed)
+                assert rule("call", p, q, 1025, 4096, mixed=mixed)
+                n = [next(k for k in range(1, 24) if rule("call", p, q, 60, 1 << k, mixed=mixed, newton64=True, max_iter=m,
+                                                          fp32_iters=m)) for m in (20, 200)]
+                assert n[1] <= n[0]  # longer chains leave the tile kernel earlier
+    assert rule("call", 1, 3, 60, 64) and rule("call", 3, 6, 60, 64)

@@ -174,7 +174,8 @@ __device__ __forceinline__ uint32_t box_mask(PTR boxes, const float p[3], float 
 // of the lanes active: 262,144 queries on a bicubic 32 x 32 net took 1199 us and now take 490, 1,000
 // queries 463 and 133 us.  One wave per SIMD without spills (273 registers): 696 us.
 // LIST: the fallback over list[0 .. *count): the (u, v) already in place is kept when it is nearer, and
-// the counts are left alone.  Otherwise it32 receives the number of leaves solved.
+// the counts are left alone.  Otherwise it32 receives the number of leaves solved.  chunk: queries per
+// wave; for a list, whose length the host doesn't know, project_chunk of that length.
 constexpr int kProjQ = 128, kProjItems = 224, kProjPer = 6;
 struct ProjWave {
     double P[3][kProjQ];
@@ -209,10 +210,22 @@ __device__ __forceinline__ void wave_lds_order() {  // LDS accesses before stay 
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Queries per wave chunk: a full pool's worth (kProjQ) once that still gives every resident wave (two
+// per SIMD) a chunk, fewer for smaller calls, whose time is the longest chain of solves in a wave.
+__host__ __device__ inline int project_chunk(size_t n, unsigned cus) {
+    const size_t c = (n / (8 * (size_t)cus) + 15) / 16 * 16;
+    return (int)(c < 16 ? 16 : c > (size_t)kProjQ ? (size_t)kProjQ : c);
+}
+
 template <int K1, int K2, bool EXACT, bool LIST>
 __global__ __launch_bounds__(256, (project_waves<K1, K2, EXACT>())) void k_project(
     GnSurfDev d_in, GnSearchDev sd, InvArgs a, const uint32_t *__restrict__ order,
-    const uint32_t *__restrict__ count, int chunk) {
+    const uint32_t *__restrict__ count, int chunk, unsigned cus) {
+    const size_t n = LIST ? (size_t)*count : a.n;
+    if constexpr (LIST) {
+        chunk = project_chunk(n, cus);
+        if ((size_t)blockIdx.x * 4 * (size_t)chunk >= n) return;  // before anything is staged
+    }
     extern __shared__ double sk[];  // EXACT: knots and reciprocal span lengths
     __shared__ __align__(16) float lbox[(((1 << (2 * (kProjLdsLevels + 1))) - 1) / 3 - 1) * 6];
     __shared__ ProjWave waves[4];
@@ -249,7 +262,6 @@ __global__ __launch_bounds__(256, (project_waves<K1, K2, EXACT>())) void k_proje
     };
     const int max_iter = a.o.max_iter;
     const double tol_step = a.o.tol_step;
-    const size_t n = LIST ? (size_t)*count : a.n;
     for (size_t q0 = ((size_t)blockIdx.x * 4 + wv) * (size_t)chunk; q0 < n;
          q0 += (size_t)gridDim.x * 4 * (size_t)chunk) {  // wave-uniform
         const int nq = (int)(n - q0 < (size_t)chunk ? n - q0 : (size_t)chunk);
@@ -631,14 +643,6 @@ __global__ void k_fb_compact(const uint8_t *__restrict__ status, size_t n, uint3
             list[atomicAdd(count, 1u)] = (uint32_t)i;
 }
 
-// Queries per wave chunk: a full pool's worth (kProjQ) once that still gives every resident wave (two
-// per SIMD) a chunk, fewer for smaller calls, whose time is the longest chain of solves in a wave.
-inline int project_chunk(size_t n) {
-    const size_t waves = (size_t)cu_count() * 8;
-    size_t c = (n / waves + 15) / 16 * 16;
-    return (int)(c < 16 ? 16 : c > (size_t)kProjQ ? (size_t)kProjQ : c);
-}
-
 struct ProjectLaunch {
     const GnSurfDev &d;
     const GnSearchDev &sd;
@@ -647,11 +651,20 @@ struct ProjectLaunch {
     hipStream_t st;
     template <int K1, int K2, bool EXACT>
     int operator()() {
-        const int chunk = count ? 16 : project_chunk(a.n);
-        const unsigned grid = grid_for(a.n, 4 * chunk, 1u << 24);
+        const unsigned cus = (unsigned)cu_count();
+        const int chunk = project_chunk(a.n, cus);
         const size_t lds = EXACT ? sizeof(double) * (2 * d.nu + 2 * d.nv + 2) : 0;
-        if (count) k_project<K1, K2, EXACT, true><<<grid, 256, lds, st>>>(d, sd, a, order, count, chunk);
-        else k_project<K1, K2, EXACT, false><<<grid, 256, lds, st>>>(d, sd, a, order, nullptr, chunk);
+        if (count) {
+            // eight workgroups per CU at most, four rounds: the list is seldom as long as the call, and a
+            // workgroup past its end costs its start (inversion and fallback of 16,000,000 queries, none of
+            // them listed: 2,442 us with a workgroup per 64 queries of the call, 1,975 with this grid; 5% of
+            // 1,000,000 listed: 1,399 and 1,221)
+            const unsigned grid = grid_for(a.n, 4 * 16, 8 * cus);
+            k_project<K1, K2, EXACT, true><<<grid, 256, lds, st>>>(d, sd, a, order, count, 0, cus);
+        } else {
+            const unsigned grid = grid_for(a.n, 4 * chunk, 1u << 23);
+            k_project<K1, K2, EXACT, false><<<grid, 256, lds, st>>>(d, sd, a, order, nullptr, chunk, cus);
+        }
         GN_HIP(hipGetLastError());
         return GN_OK;
     }

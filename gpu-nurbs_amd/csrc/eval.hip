@@ -69,8 +69,8 @@ constexpr int kLdsKnotsSmall = 512;
 // occupancy is set by registers rather than LDS.  A block takes `tiles` * 256 consecutive points and
 // the blocks start in order, so the rows are written in a narrow moving window: with a fixed grid of
 // blocks striding over the batch the waves drift apart, and 16.8M bicubic FP64 points of second order
-// took 910 us against 770, 9,999,991 FP32 points 374 against 296, 1,000,003 points of degree (5,4) and
-// third order 128 against 94.  What is left is the writes' (the same rows streamed without any
+// took 906 us against 791, 9,999,991 FP32 points 372 against 277, 1,000,003 points of degree (5,4) and
+// third order 133 against 98.  What is left is the writes' (the same rows streamed without any
 // evaluation take 515 us).
 constexpr int kRowBlock = 256;
 constexpr int kRowWaves = kRowBlock / 64;
@@ -139,25 +139,45 @@ struct EvalLaunch {
     // Tiles of 64 points per wave.  A block costs a start (its knots into LDS, the first parameters from
     // HBM), so a wave should take several; but the more of them are under way, the further apart the
     // lines written at one time, and where rows don't start on a line a line's two halves must meet in
-    // L2.  Up to eight rounds of the resident blocks, one round.  Beyond, us for 1 / 2 / 4 / 8 tiles
-    // (bicubic, second order unless said): FP64 16.8M points 889 / 770 / 855 / 901, 4.2M 197 / 175 /
-    // 165 / 166, 3,999,999 193 / 170 / 196 / 217; order 0, 4M 140 / 116 / 106 / 102; FP32 9,999,872
-    // points 231 / 209 / 191 / 191, 9,999,991 296 / 307 / 322 / 341, order 1 16M 343 / 319 / 334 / 346.
-    // FP64 patches of more than 16 entries run a block per CU: degree (5,4), third order, 1,000,003
-    // points 120 / 107 / 98 / 94.
+    // L2.  What decides is the bytes written per unit of work, per patch entry: few, and the writes wait
+    // for the waves whatever they do.  us for 1 / 2 / 4 / 8 tiles, inputs and outputs not in cache, on rows
+    // of whole lines:
+    //   FP64 under 7 (orders 0 and 1; (4,4) order 2): 16 M points, order 1 737 / 626 / 594 / 596, (4,4) order 2
+    //     1682 / 1399 / 1232 / 1162: eight; also where patches hold more than 16 entries.  (3,3) order 2 831 /
+    //     789 / 768 / 815, order 3 1118 / 1115 / 1104 / 1146: four.  (2,2) order 2 726 / 653 / 778 / 804: two; order 3
+    //     at 4,194,304 points 171 / 191 / 217 / 238: one.
+    //   FP32 (3,3) order 2, 12 M points 322 / 313 / 312 / 321, order 1, 16 M 360 / 333 / 329 / 341, (5,5) order 2 863 /
+    //     697 / 662 / 666: four.  (2,2) order 2 441 / 446 / 465 / 482: two; order 3 at 8,388,608 204 / 212 / 211 / 243:
+    //     one.
+    // and on others:
+    //   FP64 (3,3) order 2, 5,000,003 points 249 / 229 / 246 / 256: two; order 3, 4,194,305 295 / 418 / 404 / 426, (2,2)
+    //     order 2 168 / 235 / 245 / 248: one.  Patches of more than 20 entries, a block per CU: (5,4) order 3, 1,000,003
+    //     120 / 107 / 98 / 94: eight; (4,4) order 3, 4,194,305 426 / 380 / 393 / 462, 8,388,613 998 / 802 / 786 / 745: four.
+    //   FP32 (3,3) order 1, 5,000,003 108 / 98 / 93 / 94: four; (4,4) order 2, 2,000,005 78 / 74 / 77 / 85: two; (3,3)
+    //     order 2, 4,194,305 107 / 138 / 183 / 227: one.
+    // Rows a multiple of 64 MiB apart start on the same channels: four tiles lose to two, FP64 (3,3) order 2
+    // 16,777,216 points 837 / 800, FP32 482 / 462.
+    static size_t most_tiles(int entries, int order, size_t n) {
+        const size_t fields = order == 0 ? 3 : order == 1 ? 9 : order == 2 ? 18 : 30;
+        const double per = (double)(fields * sizeof(T)) / entries;  // bytes written per patch entry
+        if (n % (128 / sizeof(T)) != 0) {
+            if (sizeof(T) == 4) return per < 2.5 ? 4 : per < 4.4 ? 2 : 1;
+            if (entries > 20) return per < 9 ? 8 : 4;
+            return per < 7 ? 8 : per < 14 ? 2 : 1;
+        }
+        if (sizeof(T) == 8 && (per < 7 || entries > 16)) return 8;
+        const bool four = per < (sizeof(T) == 8 ? 15.5 : 7.8), two = per < (sizeof(T) == 8 ? 20 : 10);
+        return four && !(order >= 2 && n * sizeof(T) % ((size_t)1 << 26) == 0) ? 4 : two ? 2 : 1;
+    }
     template <int K1, int K2, int ORDER>
     int rows() {
         auto k = k_eval_rows<K1, K2, ORDER, T, TP>;
         const size_t blocks = (n + kRowBlock - 1) / kRowBlock;
         const size_t cus = (size_t)cu_count();
         const size_t resident = blocks > cus ? cus * blocks_per_cu((const void *)k, kRowBlock) : cus;
-        const bool lines = n % (128 / sizeof(T)) == 0, many = ORDER >= 2;
-        const size_t bytes = n * (ORDER == 0 ? 3 : ORDER == 1 ? 9 : ORDER == 2 ? 18 : 30) * sizeof(T);
-        size_t most = 4;
-        if (sizeof(T) == 8) most = K1 * K2 > 16 ? 8 : many && (!lines || bytes > 800000000) ? 2 : 4;
-        else if (many && !lines) most = 1;
+        const size_t most = most_tiles(K1 * K2, ORDER, n);
         size_t tiles = (blocks + resident - 1) / resident;
-        if (tiles > 8 || !lines) tiles = tiles < most ? tiles : most;
+        tiles = tiles < most ? tiles : most;
         if (tiles < n >> 31) tiles = n >> 31;  // a grid holds below 2^32 lanes
         if (tiles < 1) tiles = 1;
         const unsigned grid = (unsigned)((blocks + tiles - 1) / tiles);

@@ -1,0 +1,59 @@
+"""Scattered evaluation: a count that is no multiple of a line costs what its partial lines cost, not what a
+wrong number of tiles per wave adds; and the counts at which the rule changes its mind give the bits of
+small calls."""
+import time
+
+import pytest
+import torch
+
+import gnurbs as G
+from gnurbs import synth
+
+pytestmark = pytest.mark.gpu
+
+SMALL = 1000
+FIELDS = (3, 9, 18, 30)
+
+
+def _surface(p, q, net):
+    sd = synth.surface_G(net, net, p, q, seed=41, jitter=0.3)
+    return G.Surface(sd.p, sd.q, sd.ku, sd.kv, sd.cp, sd.w)
+
+
+@pytest.mark.parametrize("p,q,order,dtype,n", [
+    (2, 2, 3, torch.float64, 300_000), (2, 2, 2, torch.float64, 1_600_000), (3, 3, 3, torch.float64, 700_001),
+    (4, 4, 3, torch.float64, 900_001), (3, 3, 1, torch.float64, 2_200_001), (2, 2, 3, torch.float32, 600_000),
+    (2, 2, 2, torch.float32, 1_600_000), (3, 3, 2, torch.float32, 1_300_001), (4, 4, 2, torch.float32, 1_300_001),
+    (5, 5, 2, torch.float32, 1_300_001), (3, 3, 2, torch.float64, 1 << 23), (3, 3, 2, torch.float32, 1 << 24)])
+def test_bits_at_every_number_of_tiles(p, q, order, dtype, n):
+    s = _surface(p, q, 20)
+    prec = G.GN_FP64 if dtype == torch.float64 else G.GN_FP32
+    u, v = torch.rand(2, n, dtype=dtype, device="cuda", generator=torch.Generator("cuda").manual_seed(n))
+    out = torch.full((FIELDS[order], n), float("nan"), dtype=dtype, device="cuda")
+    s.Evaluate(u, v, order, precision=prec, out=out)
+    assert not torch.isnan(out).any()
+    for a in (0, n // 3, n // 2, n - SMALL):
+        one = s.Evaluate(u[a:a + SMALL].clone(), v[a:a + SMALL].clone(), order, precision=prec)
+        assert torch.equal(out[:, a:a + SMALL], one), a
+
+
+def test_partial_lines():
+    """FP32 patches of 36 entries are bound by work, not by writes: a count that is no multiple of a line
+    costs as much as one that is (a quarter more with one tile per wave)."""
+    s = _surface(5, 5, 20)
+
+    def best(n):
+        u, v = torch.rand(2, n, dtype=torch.float32, device="cuda")
+        out = torch.empty((18, n), device="cuda")
+        t = []
+        for _ in range(7):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(5):
+                s.Evaluate(u, v, 2, precision=G.GN_FP32, out=out)
+            torch.cuda.synchronize()
+            t.append(time.perf_counter() - t0)
+        return min(t[1:])
+
+    whole, part = best(12_000_032), best(12_000_007)
+    assert part < 1.12 * whole, (part, whole)

@@ -182,10 +182,11 @@ SideStreams g_side[64];  // per device, created on first use
 }  // namespace
 
 static int run_range(const GnBatchObj *objs, const GnTile *tiles, const GroupRange &gr,
-                     const GnReq *reqs, const gn_invert_opts &o, int bpc_cap, hipStream_t st) {
+                     const GnReq *reqs, const gn_invert_opts &o, int bpc_cap, hipStream_t st,
+                     bool captured = false) {
     const PathOpts limits{o.precision == GN_MIXED, (o.newton & GN_NEWTON_FP64) != 0, o.max_iter,
                           o.fp32_iters, o.fp64_tail};
-    const bool refill = batch_takes_refill(gr.grp, gr.points, limits, (size_t)cu_count());
+    const bool refill = !captured && batch_takes_refill(gr.grp, gr.points, limits, (size_t)cu_count());
     if (o.seed_mode != GN_SEED_GIVEN && (refill || o.seed_mode == GN_SEED_NEAREST_LEAF)) {
         const int rc = launch_batch_seed(objs, tiles, gr, reqs, o.seed_mode, st);
         if (rc) return rc;
@@ -250,6 +251,17 @@ static int launch_ranges(const GnBatchObj *objs, const GnTile *tiles,
         }
     }
     return rc;
+}
+
+int launch_batch_captured(const GnBatchObj *objs, const GnTile *tiles,
+                          const std::vector<GroupRange> &ranges, const GnReq *reqs,
+                          const gn_invert_opts &o, int bpc_cap, hipStream_t st) {
+    for (auto it = ranges.rbegin(); it != ranges.rend(); ++it) {
+        if (it->points == 0) continue;
+        const int rc = run_range(objs, tiles, *it, reqs, o, bpc_cap, st, true);
+        if (rc) return rc;
+    }
+    return GN_OK;
 }
 
 static int shared_side_locked(int dev) {

@@ -183,13 +183,14 @@ struct CallPlan {
     std::vector<gn::GroupRange> ranges;
 };
 
-CallPlan call_plan(const gn_batch *b, const gn_segment *segs, int nseg, int tile) {
+CallPlan call_plan(const gn_batch *b, const gn_segment *segs, int nseg, int tile, bool captured = false) {
     CallPlan c;
     size_t per[3] = {0, 0, 0}, cnt[kKeys] = {};
     int64_t most[3] = {0, 0, 0};
     for (int i = 0; i < nseg; i++) per[gn::class_group(b->cls[segs[i].obj])] += (size_t)segs[i].count;
-    const int waves = gn::batch_waves(b->bpc);
-    for (int g = 0; g < 3; g++) c.tsz[g] = gn::class_tile(per[g], waves, tile);
+    // (a captured call's list goes into kernel arguments: whole tiles keep it short)
+    const int waves = captured ? 1 : gn::batch_waves(b->bpc);
+    for (int g = 0; g < 3; g++) c.tsz[g] = captured ? std::max(tile, 64) : gn::class_tile(per[g], waves, tile);
     for (int i = 0; i < nseg; i++) {
         const int cls = b->cls[segs[i].obj], g = gn::class_group(cls);
         cnt[gn::class_order(cls)] += (size_t)((segs[i].count + c.tsz[g] - 1) / c.tsz[g]);
@@ -226,21 +227,43 @@ void write_image(const gn_batch *b, const gn_segment *segs, int nseg, const Call
 
 void free_image_host(void *p) { delete static_cast<std::vector<char> *>(p); }
 
+// Under stream capture the image travels in the arguments of kernel nodes, which the graph keeps, to a
+// buffer that the graph allocates and frees: a replay reads nothing of the host's and nothing that another
+// launch may be given (the kernels take no counter slots, and the shared side streams stay out of the
+// capture).  A copy node from the call's host image would read freed memory from the second replay on.
+int run_captured(gn_batch *b, const gn_segment *segs, int nseg, const GnReq &req, const gn_invert_opts &o,
+                 int tile, int bpc, hipStream_t st) {
+    const CallPlan c = call_plan(b, segs, nseg, tile, true);
+    if (c.ntiles == 0) return GN_OK;
+    std::vector<char> img((c.bytes + 15) & ~(size_t)15);
+    write_image(b, segs, nseg, c, req, img.data());
+    char *d = nullptr;
+    GN_HIP(hipMallocAsync((void **)&d, img.size(), st));
+    int rc = gn::launch_stage_args(img.data(), d, img.size(), st);
+    if (!rc)
+        rc = gn::launch_batch_captured(b->d_objs, (const GnTile *)d, c.ranges,
+                                       (const GnReq *)(d + c.req_off), o, bpc, st);
+    const hipError_t e = hipFreeAsync(d, st);
+    if (!rc && e != hipSuccess) rc = gn::hip_fail(e, "hipFreeAsync(tiles)");
+    return rc;
+}
+
 // The call image is written into pinned staging of the batch's pool and a small kernel carries it to
 // the device, so a call neither allocates nor waits.  (A stream-ordered allocation, a copy from
 // pageable memory and a host callback that freed it put 0.4 ms of host time and a bubble before the
-// first kernel: 256 surfaces and 1.09M points, 897 us for a call on an idle device.)  A call under stream
-// capture, or without a staging buffer, takes the stream-ordered form.
+// first kernel: 256 surfaces and 1.09M points, 897 us for a call on an idle device.)  A call without a
+// staging buffer takes that stream-ordered form.
 int run_batch(gn_batch *b, const gn_segment *segs, int nseg, const double *x, const double *y,
               const double *z, size_t n, const gn_invert_opts &o, double *u, double *v,
               uint8_t *status, uint8_t *it32, uint8_t *it64, int tile, int bpc, hipStream_t st) {
     (void)n;
     const GnReq req{x, y, z, u, v, status, it32, it64};
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess) (void)hipGetLastError();  // (the null stream, beside a capture)
+    if (cs != hipStreamCaptureStatusNone) return run_captured(b, segs, nseg, req, o, tile, bpc, st);
     const CallPlan c = call_plan(b, segs, nseg, tile);
     if (c.ntiles == 0) return GN_OK;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    const bool capturing = hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone;
-    CallBuf *buf = capturing ? nullptr : b->calls.take(c.bytes + 16);
+    CallBuf *buf = b->calls.take(c.bytes + 16);
     if (buf) {
         write_image(b, segs, nseg, c, req, buf->h);
         int rc = gn::launch_stage_copy(buf->h_dev, buf->d, c.bytes, st);

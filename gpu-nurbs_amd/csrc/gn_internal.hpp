@@ -271,6 +271,11 @@ int launch_batch_invert(const GnBatchObj *objs, const GnTile *tiles,
                         const SideStreams *side = nullptr,
                         const std::function<int(hipStream_t)> &beside = {},
                         std::vector<std::pair<int, hipEvent_t>> *group_done = nullptr);
+// The same into a capture that outlives the call: one group after the other on st, without the shared
+// side streams and without launches that take counter slots from the device's ring.
+int launch_batch_captured(const GnBatchObj *objs, const GnTile *tiles,
+                          const std::vector<GroupRange> &ranges, const GnReq *reqs,
+                          const gn_invert_opts &o, int bpc_cap, hipStream_t st);
 // Seeds of a group range's points into their requests' u, v, and the range's persistent launches from
 // them (batch_refill.hip).
 int launch_batch_seed(const GnBatchObj *objs, const GnTile *tiles, const GroupRange &gr,
@@ -315,6 +320,9 @@ class PoolScope {
 // ordinary kernel on st; both buffers 16-byte aligned and readable/writable to bytes rounded up
 // to 16.
 int launch_stage_copy(const void *src, void *dst, size_t bytes, hipStream_t st);
+// Copies host memory to device memory (16-byte aligned, a multiple of 16 bytes) in the arguments of
+// kernels, for captures: the graph's nodes hold the bytes.
+int launch_stage_args(const char *src, char *dst, size_t bytes, hipStream_t st);
 int launch_copy_results(const double *su, const double *sv, const uint8_t *ss, size_t n, double *du,
                         double *dv, uint8_t *ds, hipStream_t st);
 // Argument checks of gn_invert (a failing check sets the thread's error message).

@@ -11,6 +11,7 @@
 //   - a copy kernel for small host-to-device images (the server's step tables).
 //   - the compute-unit count used to size persistent grids.
 #include <atomic>
+#include <cstring>
 #include <mutex>
 #include <unordered_map>
 
@@ -109,6 +110,27 @@ int launch_stage_copy(const void *src, void *dst, size_t bytes, hipStream_t st) 
     k_stage_copy<<<(unsigned)(blocks < 1024 ? blocks : 1024), 256, 0, st>>>(
         (const uint4 *)src, (uint4 *)dst, n);
     GN_HIP(hipGetLastError());
+    return GN_OK;
+}
+
+// 3.5 KB of kernel arguments (a launch takes 4 KB); a lane copies one 16-byte vector.
+struct StageArgs {
+    uint4 v[224];
+};
+__global__ __launch_bounds__(256) void k_stage_args(StageArgs a, uint4 *__restrict__ dst, int n) {
+    const int i = threadIdx.x;
+    if (i < n) dst[i] = a.v[i];
+}
+
+int launch_stage_args(const char *src, char *dst, size_t bytes, hipStream_t st) {
+    for (size_t at = 0; at < bytes; at += sizeof(StageArgs)) {
+        const size_t part = bytes - at < sizeof(StageArgs) ? bytes - at : sizeof(StageArgs);
+        StageArgs a;
+        std::memset(&a, 0, sizeof(a));
+        std::memcpy(&a, src + at, part);
+        k_stage_args<<<1, 256, 0, st>>>(a, (uint4 *)(dst + at), (int)(part / 16));
+        GN_HIP(hipGetLastError());
+    }
     return GN_OK;
 }
 

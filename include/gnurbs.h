@@ -268,9 +268,10 @@ size_t gn_batch_device_bytes(const gn_batch *b);
 int gn_batch_set_shape(gn_batch *b, int tile_points, int blocks_per_cu);
 int gn_batch_get_shape(const gn_batch *b, int *tile_points, int *blocks_per_cu);
 /* Inverts the points of all segments (device arrays x, y, z, u, v, status of length n) with one
- * launch per group of degree classes (a seed launch and persistent ones for groups of many points); seeds: GN_SEED_GREEDY_LEAF, GN_SEED_NEAREST_LEAF,
- * GN_SEED_GREEDY_STEP, GN_SEED_GRID_STEP (each point on its own surface's tree or grid) or
- * GN_SEED_GIVEN. */
+ * launch per group of degree classes, or a seed launch and persistent ones for groups of many points;
+ * seeds: GN_SEED_GREEDY_LEAF, GN_SEED_NEAREST_LEAF, GN_SEED_GREEDY_STEP, GN_SEED_GRID_STEP (each point
+ * on its own surface's tree or grid) or GN_SEED_GIVEN.  In a caller's own stream capture the graph keeps
+ * the segments of the call; it may be replayed any number of times while the batch lives. */
 int gn_batch_invert(gn_batch *b, const gn_segment *segs, int nseg, const double *x,
                     const double *y, const double *z, size_t n, const gn_invert_opts *opts,
                     double *u, double *v, uint8_t *status, gn_stream stream);

@@ -26,6 +26,7 @@ struct CallBuf {
     void *h_dev = nullptr;  // h's device-side address
     size_t cap = 0;
     hipEvent_t ev = nullptr;
+    hipStream_t st = nullptr;  // the stream of the call in flight
     bool taken = false, pending = false;
     unsigned long long seq = 0;  // order of use
 };
@@ -34,9 +35,10 @@ struct CallBuf {
 class CallPool {
   public:
     static constexpr size_t kMax = 8;
-    // A buffer of at least `bytes`.  With kMax calls in flight it waits for the oldest of them; null if
-    // other threads are enqueuing calls with all of them, or none could be allocated.
-    CallBuf *take(size_t bytes) {
+    // A buffer of at least `bytes` for a call on st.  With all buffers in flight it waits for the oldest
+    // call of the same stream; null if there is none (another stream's work may take any time, or wait
+    // for this host thread), or if no buffer could be allocated.
+    CallBuf *take(size_t bytes, hipStream_t st) {
         CallBuf *best = nullptr;
         {
             std::lock_guard<std::mutex> lk(mu_);
@@ -62,9 +64,10 @@ class CallPool {
             }
             if (!best)
                 for (CallBuf *b : all_)
-                    if (!b->taken && (!best || b->seq < best->seq)) best = b;
+                    if (!b->taken && b->st == st && (!best || b->seq < best->seq)) best = b;
             if (!best) return nullptr;
             best->taken = true;
+            best->st = st;
             best->seq = ++seq_;
         }
         if (best->pending && hipEventSynchronize(best->ev) != hipSuccess) (void)hipGetLastError();
@@ -78,7 +81,7 @@ class CallPool {
     }
     // A first buffer, made with the batch rather than in its first call; calls do without if it fails.
     void reserve(size_t bytes) {
-        CallBuf *b = take(bytes);
+        CallBuf *b = take(bytes, nullptr);
         if (b) b->taken = false;
     }
     // After the call's work has been enqueued on st.
@@ -263,7 +266,7 @@ int run_batch(gn_batch *b, const gn_segment *segs, int nseg, const double *x, co
     if (cs != hipStreamCaptureStatusNone) return run_captured(b, segs, nseg, req, o, tile, bpc, st);
     const CallPlan c = call_plan(b, segs, nseg, tile);
     if (c.ntiles == 0) return GN_OK;
-    CallBuf *buf = b->calls.take(c.bytes + 16);
+    CallBuf *buf = b->calls.take(c.bytes + 16, st);
     if (buf) {
         write_image(b, segs, nseg, c, req, buf->h);
         int rc = gn::launch_stage_copy(buf->h_dev, buf->d, c.bytes, st);

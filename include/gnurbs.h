@@ -270,7 +270,8 @@ int gn_batch_get_shape(const gn_batch *b, int *tile_points, int *blocks_per_cu);
 /* Inverts the points of all segments (device arrays x, y, z, u, v, status of length n) with one
  * launch per group of degree classes, or a seed launch and persistent ones for groups of many points;
  * seeds: GN_SEED_GREEDY_LEAF, GN_SEED_NEAREST_LEAF, GN_SEED_GREEDY_STEP, GN_SEED_GRID_STEP (each point
- * on its own surface's tree or grid) or GN_SEED_GIVEN.  In a caller's own stream capture the graph keeps
+ * on its own surface's tree or grid) or GN_SEED_GIVEN.  With eight calls of a batch in flight the next
+ * one on the same stream first waits for the oldest of them.  In a caller's own stream capture the graph keeps
  * the segments of the call; it may be replayed any number of times while the batch lives. */
 int gn_batch_invert(gn_batch *b, const gn_segment *segs, int nseg, const double *x,
                     const double *y, const double *z, size_t n, const gn_invert_opts *opts,

@@ -98,37 +98,49 @@ class CallPool {
     // The device must be idle.
     void clear() {
         for (CallBuf *b : all_) {
-            release(b);
+            release(b->h, b->d);
             (void)hipEventDestroy(b->ev);
             delete b;
         }
+        for (const Outgrown &o : outgrown_) release(o.h, o.d);
         all_.clear();
+        outgrown_.clear();
     }
 
   private:
-    static void release(CallBuf *b) {
-        if (b->h) (void)hipHostFree(b->h);
-        if (b->d) (void)hipFree(b->d);
-        b->h = b->d = nullptr;
-        b->h_dev = nullptr;
-        b->cap = 0;
+    struct Outgrown {
+        char *h, *d;
+    };
+    static void release(char *h, char *d) {
+        if (h) (void)hipHostFree(h);
+        if (d) (void)hipFree(d);
     }
-    static bool grow(CallBuf *b, size_t bytes) {
-        release(b);
+    // A free waits for the whole device: what a buffer outgrew stays until the batch is destroyed.  (Sizes
+    // double, so that is less than the buffer's own size.)
+    bool grow(CallBuf *b, size_t bytes) {
         size_t cap = 1 << 16;
         while (cap < bytes) cap <<= 1;
-        if (hipHostMalloc((void **)&b->h, cap, hipHostMallocCoherent) != hipSuccess ||
-            hipHostGetDevicePointer(&b->h_dev, b->h, 0) != hipSuccess ||
-            hipMalloc((void **)&b->d, cap) != hipSuccess) {
+        CallBuf n;
+        if (hipHostMalloc((void **)&n.h, cap, hipHostMallocCoherent) != hipSuccess ||
+            hipHostGetDevicePointer(&n.h_dev, n.h, 0) != hipSuccess ||
+            hipMalloc((void **)&n.d, cap) != hipSuccess) {
             (void)hipGetLastError();
-            release(b);
+            release(n.h, n.d);
             return false;
         }
+        if (b->h) {
+            std::lock_guard<std::mutex> lk(mu_);
+            outgrown_.push_back(Outgrown{b->h, b->d});
+        }
+        b->h = n.h;
+        b->h_dev = n.h_dev;
+        b->d = n.d;
         b->cap = cap;
         return true;
     }
     std::mutex mu_;
     std::vector<CallBuf *> all_;
+    std::vector<Outgrown> outgrown_;
     unsigned long long seq_ = 0;
 };
 

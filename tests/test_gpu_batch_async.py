@@ -91,3 +91,26 @@ def test_eight_calls_in_flight_do_not_hold_up_another_stream(work):
     _check(outs, ref)
     assert whole > 0.3 and other < 0.5 * whole, (other, whole)
     b.close()
+
+
+def test_a_longer_list_does_not_wait_for_the_device(work):
+    """All staging buffers are too small for the call's list."""
+    s, P, o = work
+    b = G.Batch([s])
+    b.set_shape(64, 0)
+    ref = [t.clone() for t in b.invert(_segs(3), *P, o)]
+    outs = _outs(9)
+    s1, s2 = _streams()
+    _sleep(s1, 0.05)
+    for out in outs[:8]:
+        b.invert(_segs(3), *P, o, out=out, stream=s1)
+    _check(outs[:8], ref)
+    t0 = _sleep(s1, 0.5)
+    b.invert(_segs(50_000), *P, o, out=outs[8], stream=s2)
+    s2.synchronize()
+    other = time.perf_counter() - t0
+    torch.cuda.synchronize()
+    whole = time.perf_counter() - t0
+    _check(outs, ref)
+    assert whole > 0.3 and other < 0.5 * whole, (other, whole)
+    b.close()

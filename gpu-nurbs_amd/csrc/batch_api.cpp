@@ -95,6 +95,11 @@ class CallPool {
         b->pending = rec;
         b->taken = false;
     }
+    // Device memory held.
+    size_t device_bytes() const {
+        std::lock_guard<std::mutex> lk(mu_);
+        return bytes_;
+    }
     // The device must be idle.
     void clear() {
         for (CallBuf *b : all_) {
@@ -105,6 +110,7 @@ class CallPool {
         for (const Outgrown &o : outgrown_) release(o.h, o.d);
         all_.clear();
         outgrown_.clear();
+        bytes_ = 0;
     }
 
   private:
@@ -128,19 +134,19 @@ class CallPool {
             release(n.h, n.d);
             return false;
         }
-        if (b->h) {
-            std::lock_guard<std::mutex> lk(mu_);
-            outgrown_.push_back(Outgrown{b->h, b->d});
-        }
+        std::lock_guard<std::mutex> lk(mu_);
+        if (b->h) outgrown_.push_back(Outgrown{b->h, b->d});
+        bytes_ += cap;
         b->h = n.h;
         b->h_dev = n.h_dev;
         b->d = n.d;
         b->cap = cap;
         return true;
     }
-    std::mutex mu_;
+    mutable std::mutex mu_;
     std::vector<CallBuf *> all_;
     std::vector<Outgrown> outgrown_;
+    size_t bytes_ = 0;
     unsigned long long seq_ = 0;
 };
 
@@ -351,7 +357,7 @@ int batch_view(const gn_batch *b, const GnBatchObj **objs, int *count, std::vect
     *cls = b->cls;
     *tile = b->tile;
     *bpc = b->bpc;
-    *bytes = b->bytes;
+    *bytes = b->bytes + b->calls.device_bytes();
     return GN_OK;
 }
 }  // namespace gn
@@ -469,7 +475,9 @@ int gn_batch_destroy(gn_batch *b) {
     return GN_OK;
 }
 
-size_t gn_batch_device_bytes(const gn_batch *b) { return b ? b->bytes : 0; }
+size_t gn_batch_device_bytes(const gn_batch *b) {
+    return b ? b->bytes + b->calls.device_bytes() : 0;
+}
 
 int gn_batch_set_shape(gn_batch *b, int tile_points, int blocks_per_cu) {
     if (!b) return fail(GN_EINVAL, "null batch");

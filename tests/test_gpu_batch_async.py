@@ -114,3 +114,22 @@ def test_a_longer_list_does_not_wait_for_the_device(work):
     _check(outs, ref)
     assert whole > 0.3 and other < 0.5 * whole, (other, whole)
     b.close()
+
+
+def test_device_bytes_count_the_staging(work):
+    """The memory of a batch's staging buffers, from its creation on and as they grow."""
+    s, P, o = work
+    free = torch.cuda.mem_get_info()[0]
+    b = G.Batch([s])
+    size = lambda: int(G.lib().gn_batch_device_bytes(b._h))  # noqa: E731
+    first = size()
+    assert abs((free - torch.cuda.mem_get_info()[0]) - first) <= 8 << 20  # (allocations are rounded up)
+    b.set_shape(64, 0)
+    b.invert(_segs(50_000), *P, o)
+    torch.cuda.synchronize()
+    assert size() - first >= 50_000 * 32
+    grown = size()
+    b.invert(_segs(50_000), *P, o)
+    torch.cuda.synchronize()
+    assert size() == grown
+    b.close()

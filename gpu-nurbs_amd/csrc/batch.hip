@@ -183,10 +183,10 @@ SideStreams g_side[64];  // per device, created on first use
 
 static int run_range(const GnBatchObj *objs, const GnTile *tiles, const GroupRange &gr,
                      const GnReq *reqs, const gn_invert_opts &o, int bpc_cap, hipStream_t st,
-                     bool captured = false) {
+                     bool several, bool captured = false) {
     const PathOpts limits{o.precision == GN_MIXED, (o.newton & GN_NEWTON_FP64) != 0, o.max_iter,
                           o.fp32_iters, o.fp64_tail};
-    const bool refill = !captured && batch_takes_refill(gr.grp, gr.points, limits, (size_t)cu_count());
+    const bool refill = !captured && batch_takes_refill(gr.grp, gr.points, several, limits, (size_t)cu_count());
     if (o.seed_mode != GN_SEED_GIVEN && (refill || o.seed_mode == GN_SEED_NEAREST_LEAF)) {
         const int rc = launch_batch_seed(objs, tiles, gr, reqs, o.seed_mode, st);
         if (rc) return rc;
@@ -207,7 +207,7 @@ static int launch_ranges(const GnBatchObj *objs, const GnTile *tiles,
                          const SideStreams &ss, const std::function<int(hipStream_t)> &beside,
                          std::vector<std::pair<int, hipEvent_t>> *group_done) {
     if (ranges.size() == 1 && !beside)  // one group, nothing beside it: no fork
-        return run_range(objs, tiles, ranges[0], reqs, o, bpc_cap, st);
+        return run_range(objs, tiles, ranges[0], reqs, o, bpc_cap, st, false);
     if (ranges.size() > (size_t)kSideStreams)
         return fail(GN_EDEVICE, "more group ranges than side streams (tiles not sorted by class)");
     GN_HIP(hipEventRecord(ss.fork, st));
@@ -222,7 +222,7 @@ static int launch_ranges(const GnBatchObj *objs, const GnTile *tiles,
         const GroupRange &gr = *it;
         if (gr.points == 0) continue;
         if (own && it == ranges.rbegin()) {
-            rc = run_range(objs, tiles, gr, reqs, o, bpc_cap, st);
+            rc = run_range(objs, tiles, gr, reqs, o, bpc_cap, st, ranges.size() > 1);
             if (rc) break;
             continue;
         }
@@ -231,7 +231,7 @@ static int launch_ranges(const GnBatchObj *objs, const GnTile *tiles,
             rc = hip_fail(e, "hipStreamWaitEvent(fork)");
             break;
         }
-        rc = run_range(objs, tiles, gr, reqs, o, bpc_cap, ss.s[k]);
+        rc = run_range(objs, tiles, gr, reqs, o, bpc_cap, ss.s[k], ranges.size() > 1);
         const hipError_t ej = hipEventRecord(ss.join[k], ss.s[k]);
         if (ej != hipSuccess) {
             if (!rc) rc = hip_fail(ej, "hipEventRecord(join)");
@@ -258,7 +258,7 @@ int launch_batch_captured(const GnBatchObj *objs, const GnTile *tiles,
                           const gn_invert_opts &o, int bpc_cap, hipStream_t st) {
     for (auto it = ranges.rbegin(); it != ranges.rend(); ++it) {
         if (it->points == 0) continue;
-        const int rc = run_range(objs, tiles, *it, reqs, o, bpc_cap, st, true);
+        const int rc = run_range(objs, tiles, *it, reqs, o, bpc_cap, st, false, true);
         if (rc) return rc;
     }
     return GN_OK;

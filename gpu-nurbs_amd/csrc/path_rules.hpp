@@ -66,7 +66,10 @@ inline bool call_takes_tile(int p, int q, size_t knots, size_t n, const PathOpts
 //     times that: tile; (5,5) 1.16 / 1.01 at 4 rounds, 1.02 / 0.85 at 16.  20 and 3 (29): group 0 1.08 / 0.84 at
 //     1,048,576; (5,5) 1.13 / 0.89 at two rounds, 0.90 / 0.58 at 16.  6 and 12 (42): (3,3) 1.16 / 1.01 at two,
 //     0.96 / 0.77 at 8.  30 and 40 (150): (3,3) 1.01 / 0.93 at half a round, 0.68 / 0.45 at 8.
-inline bool batch_takes_refill(int grp, size_t points, const PathOpts &o, size_t cus) {
+// Beside other groups a persistent launch, which fills the chip, costs more: uneven surfaces of all three
+// groups, the second group by refill and by tile, us: 236,000 points (3.6 rounds) 340 / 287 for a limit of 42, 339 /
+// 287 for 29; 448,000 (6.8 rounds) 473 / 492 for 29, 398 / 365 for 15; 1,068,000 798 / 791 for 15.
+inline bool batch_takes_refill(int grp, size_t points, bool several, const PathOpts &o, size_t cus) {
     const size_t limit = chain_limit(o);
     const size_t waves = o.mixed ? (grp == 0 ? 8 : 4) : (size_t)(4 - grp), round = 64 * waves * cus;
     if (!o.mixed) {
@@ -74,7 +77,7 @@ inline bool batch_takes_refill(int grp, size_t points, const PathOpts &o, size_t
         return points > (limit > 20 ? round / 2 : grp == 1 && !o.newton64 ? 3 * round : round);
     }
     if (grp == 0 && limit <= 32) return false;
-    return points * limit > round * (grp == 0 ? 84 : 64);
+    return points * limit > round * (grp == 0 ? 84 : several ? 160 : 64);
 }
 
 }  // namespace gn

@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 DEGREES = [(p, q) for p in range(2, 6) for q in range(2, 6)] + [(1, 3), (6, 2)]
 # points of group 0, 1 and 2 (patches of at most 16 entries, of at most 25, others): above the rule's
 # bounds for PLAIN with a Newton bit and for MIXED (test_path_rules.py)
-POINTS = [82_000, 41_003, 33_001]
+POINTS = [82_000, 72_003, 71_001]
 PLAIN = dict(max_iter=25)
 MIXED = dict(precision=G.GN_MIXED, fp32_iters=30, fp64_tail=40, tol_step32=3e-5, tol_step=1e-10, tol_quad=1e-10)
 SEEDS = [G.SEED_GREEDY_LEAF, G.SEED_GREEDY_STEP, G.SEED_GRID_STEP, G.SEED_NEAREST_LEAF, G.SEED_GIVEN]

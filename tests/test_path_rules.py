@@ -16,12 +16,12 @@ DRIVER = r"""
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
-// batch GRP POINTS | call P Q KNOTS POINTS, then MIXED NEWTON64 MAX_ITER FP32_ITERS FP64_TAIL: 1 if persistent
+// batch GRP POINTS SEVERAL | call P Q KNOTS POINTS, then MIXED NEWTON64 MAX_ITER FP32_ITERS FP64_TAIL: 1 if persistent
 int main(int argc, char **argv) {
     auto n = [&](int k) { return (size_t)atoll(argv[k]); };
     const int at = argc - 5;
     const gn::PathOpts o{n(at) != 0, n(at + 1) != 0, (int)n(at + 2), (int)n(at + 3), (int)n(at + 4)};
-    if (!strcmp(argv[1], "batch")) printf("%d", (int)gn::batch_takes_refill((int)n(2), n(3), o, 256));
+    if (!strcmp(argv[1], "batch")) printf("%d", (int)gn::batch_takes_refill((int)n(2), n(3), n(4) != 0, o, 256));
     else printf("%d", (int)!gn::call_takes_tile((int)n(2), (int)n(3), n(4), n(5), o, 256));
     return 0;
 }
@@ -45,21 +45,24 @@ def rule(tmp_path_factory):
 @pytest.mark.parametrize("grp", [0, 1, 2])
 def test_batches_of_the_refill_tests_are_persistent(rule, grp):
     n = sum(c for c, (p, q) in zip(batch_refill.counts(), batch_refill.DEGREES) if batch_refill.group(p, q) == grp)
-    assert rule("batch", grp, n, newton64=True, max_iter=batch_refill.PLAIN["max_iter"])
+    assert rule("batch", grp, n, 1, newton64=True, max_iter=batch_refill.PLAIN["max_iter"])
     m = batch_refill.MIXED
-    assert rule("batch", grp, n, mixed=True, fp32_iters=m["fp32_iters"], fp64_tail=m["fp64_tail"])
+    assert rule("batch", grp, n, 1, mixed=True, fp32_iters=m["fp32_iters"], fp64_tail=m["fp64_tail"])
 
 
 def test_batch_rule(rule):
     """Up to half a round of waves every chain is short enough to wait for; long chains in many rounds are not."""
+    waves = {True: (8, 4, 4), False: (4, 3, 2)}
+    long = dict(newton64=True, max_iter=100, fp32_iters=30, fp64_tail=40)
     for grp in (0, 1, 2):
-        waves = {True: (8, 4, 4), False: (4, 3, 2)}
         for mixed in (False, True):
             half = 32 * 256 * waves[mixed][grp]
-            assert not rule("batch", grp, half // 2, mixed=mixed, newton64=True, max_iter=100, fp32_iters=30, fp64_tail=40)
-            assert rule("batch", grp, 8 * half, mixed=mixed, newton64=True, max_iter=100, fp32_iters=30, fp64_tail=40)
-    assert not rule("batch", 0, 1 << 24, max_iter=20) and rule("batch", 0, 1 << 24, max_iter=21)
-    assert not rule("batch", 0, 1 << 24, mixed=True, fp32_iters=6, fp64_tail=3)
+            for several in (0, 1):
+                assert not rule("batch", grp, half // 2, several, mixed=mixed, **long)
+                assert rule("batch", grp, 8 * half, several, mixed=mixed, **long)
+    for several in (0, 1):
+        assert not rule("batch", 0, 1 << 24, several, max_iter=20) and rule("batch", 0, 1 << 24, several, max_iter=21)
+        assert not rule("batch", 0, 1 << 24, several, mixed=True, fp32_iters=6, fp64_tail=3)
 
 
 def _call(rule, p, q, n, opts, newton64=True):

@@ -43,12 +43,11 @@ constexpr int group_patch_vecs() {
 // small nets, so nothing is shared between waves; the bound is one point's chain of iterations, and
 // past a few rounds of waves their VALU and patch loads.  Before, a seed launch, persistent FP32 and
 // FP64 launches that claimed tiles and refilled stopped lanes: one launch instead of three per
-// group, and no drain where a wave's next tile is of another class.  Uneven batches, whole call
-// before and now: 16 surfaces 79,297 points mixed 179 -> 105 us, 64 surfaces 55,347 points FP64 415
-// -> 249, 256 surfaces 1,090,341 points mixed 464 -> 407 and FP64 1,384 -> 1,173, 1,024 surfaces
-// 4.9 M points mixed 1,763 -> 1,527 and FP64 6,362 -> 5,193.  (The knots in LDS: no gain at 55,347
-// points, 10% slower at 1,090,341, fewer waves.)
-
+// group, and no drain where a wave's next tile is of another class.  Uneven batches, every group on the
+// persistent kernels and on this one, mixed with 6 and 3 steps: 16 surfaces 79,297 points 107 and 69 us, 64
+// surfaces 221,393 points 159 and 121, 256 surfaces 1,090,341 points 428 and 365, 1,024 surfaces 4.9 M
+// points 1,640 and 1,600; FP64, 20 Gauss-Newton steps, 256 surfaces 1,404 and 1,274.  (The knots in LDS:
+// no gain at 55,347 points, 10% slower at 1,090,341, fewer waves.)
 template <int GRP, bool MIXED, bool NEWTON32, bool NEWTON64>
 __global__ __launch_bounds__(64, 1) void k_batch_tile(BatchTileArgs a) {
     __shared__ float4 patches[group_patch_vecs<GRP, MIXED>()];

@@ -168,8 +168,8 @@ struct gn_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     char *d_buf = nullptr;  // tile list + request table of the captured call
-    // the claim-counter slots baked into the graph: its own, so no eager launch is ever given
-    // them (each replay leaves them zeroed for the next)
+    // the claim-counter slots of persistent launches baked into the graph: its own, so no eager launch is
+    // ever given them (each replay leaves them zeroed for the next)
     unsigned long long *d_ctr = nullptr;
 };
 
@@ -612,7 +612,7 @@ int gn_batch_graph_create(gn_batch *b, const gn_segment *segs, int nseg, const d
     write_image(b, segs, nseg, plan, req, img.data());
     gn_graph *g = new gn_graph();
     hipStream_t st = (hipStream_t)stream;
-    // one slot per persistent launch: one per class group and precision phase
+    // a slot per persistent launch: at most one per class group and precision phase
     gn::SlotPool pool;
     pool.nslots = (int)plan.ranges.size() * (o.precision == GN_MIXED ? 2 : 1);
     const size_t ctr_bytes = sizeof(unsigned long long) * gn::slot_words() * (pool.nslots ? pool.nslots : 1);

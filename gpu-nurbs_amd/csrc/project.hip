@@ -169,9 +169,10 @@ __device__ __forceinline__ uint32_t box_mask(PTR boxes, const float p[3], float 
 // comes in the query's order; a leaf whose box is farther cannot hold a nearer point, so solving it
 // ahead of its turn changes no result.
 // What bounds the kernel is FP64 evaluation (one step of up to 64 solves: 2.9 us per wave at two waves
-// per SIMD, 40 lanes active on average) and then the walks, about a fifth; for small calls the longest
+// per SIMD; over the whole kernel 26 of 64 lanes are active per VALU instruction) and then the walks, about a
+// fifth; for small calls the longest
 // chain of solves.  One query per lane, its solves gathered into rounds with the other lanes', kept 19%
-// of the lanes active: 262,144 queries on a bicubic 32 x 32 net took 1199 us and now take 490, 1,000
+// of the lanes active: 262,144 queries on a bicubic 32 x 32 net took 1194 us and now take 501, 1,000
 // queries 463 and 133 us.  One wave per SIMD without spills (273 registers): 696 us.
 // LIST: the fallback over list[0 .. *count): the (u, v) already in place is kept when it is nearer, and
 // the counts are left alone.  Otherwise it32 receives the number of leaves solved.  chunk: queries per
@@ -557,8 +558,8 @@ __global__ __launch_bounds__(256, (project_waves<K1, K2, EXACT>())) void k_proje
 // writes each query's index to its key's next slot within the block's own range of `order`.  Keys stay
 // in registers between the two passes and the block's loads are issued together: with blocks of 65,536
 // read twice in sequence, four workgroups took 103 us for 262,144 queries.  The
-// order within one key is unspecified; each query's result does not depend on it (project_point
-// is per query).
+// order within one key is unspecified; each query's result is its own and does not depend
+// on it.
 constexpr int kOrdThreads = 1024;
 constexpr int kOrdPer = 16;  // queries per thread
 constexpr size_t kOrdBlock = (size_t)kOrdPer * kOrdThreads;

@@ -210,7 +210,7 @@ int gn_server::launch_step(Slot &sl) {
     if (crc) return crc;
     const GnReq *d_rq = (const GnReq *)sl.d_stage;
     const GnTile *d_tl = (const GnTile *)(sl.d_stage + toff);
-    // surface groups (seeds and precision phases) on the slot's side streams, curves on the
+    // surface groups on the slot's side streams, curves on the
     // slot's stream beside them; all joined back before the step's event
     std::function<int(hipStream_t)> curves;
     if (nc)

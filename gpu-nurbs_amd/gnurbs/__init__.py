@@ -663,7 +663,7 @@ class Graph:
 
 
 class Batch:
-    """Many surfaces packed for one persistent inversion launch (gn_batch).  Every surface must
+    """Many surfaces packed for one inversion call (gn_batch).  Every surface must
     have its tree built."""
 
     def __init__(self, surfaces, stream=None):

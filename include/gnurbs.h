@@ -244,7 +244,7 @@ int gn_invert_noalloc(const gn_surface *s, const double *x, const double *y, con
                       size_t n, const gn_invert_opts *opts, double *u_out, double *v_out,
                       uint8_t *status, gn_stream stream);
 
-/* ---- batched inversion: many surfaces in one persistent launch ---------------------------- */
+/* ---- batched inversion: many surfaces in one call ------------------------------------------ */
 
 /* A run of points that belong to one object of a batch: points start .. start+count-1 of the
  * query arrays are inverted on object `obj` (index into the batch's surface list). */

@@ -270,14 +270,6 @@ static int shared_side_locked(int dev) {
     return rc;
 }
 
-int batch_prepare() {
-    int dev = 0;
-    GN_HIP(hipGetDevice(&dev));
-    if (dev < 0 || dev >= 64) return fail(GN_EDEVICE, "device index out of range");
-    std::lock_guard<std::mutex> lk(g_side_mu);
-    return shared_side_locked(dev);
-}
-
 int launch_batch_invert(const GnBatchObj *objs, const GnTile *tiles,
                         const std::vector<GroupRange> &ranges, const GnReq *reqs,
                         const gn_invert_opts &o, int bpc_cap, hipStream_t st,

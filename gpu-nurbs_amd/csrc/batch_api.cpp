@@ -605,7 +605,6 @@ int gn_batch_graph_create(gn_batch *b, const gn_segment *segs, int nseg, const d
     if ((rc = check_segments(b, segs, nseg, n))) return rc;
     if (n && (!x || !y || !z || !u || !v || !status)) return fail(GN_EINVAL, "null buffer");
     if ((rc = gn::ensure_runtime())) return rc;
-    if ((rc = gn::batch_prepare())) return rc;
     const GnReq req{x, y, z, u, v, status, nullptr, nullptr};
     const CallPlan plan = call_plan(b, segs, nseg, b->tile);
     std::vector<char> img(plan.bytes);
@@ -629,8 +628,19 @@ int gn_batch_graph_create(gn_batch *b, const gn_segment *segs, int nseg, const d
         return gn::hip_fail(e, "graph tile list / counter slots");
     }
     pool.ctr = g->d_ctr;
+    // side streams of its own: they stay in the capture until it ends, and a call of another thread that
+    // was given the shared ones meanwhile would fail
+    gn::SideStreams side;
+    if ((rc = gn::side_streams_create(&side))) {
+        gn::side_streams_destroy(&side);
+        (void)hipFree(g->d_buf);
+        (void)hipFree(g->d_ctr);
+        delete g;
+        return rc;
+    }
     e = hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) {
+        gn::side_streams_destroy(&side);
         (void)hipFree(g->d_buf);
         (void)hipFree(g->d_ctr);
         delete g;
@@ -639,9 +649,10 @@ int gn_batch_graph_create(gn_batch *b, const gn_segment *segs, int nseg, const d
     {
         gn::PoolScope scope(&pool);
         rc = gn::launch_batch_invert(b->d_objs, (const GnTile *)g->d_buf, plan.ranges,
-                                     (const GnReq *)(g->d_buf + plan.req_off), o, b->bpc, st);
+                                     (const GnReq *)(g->d_buf + plan.req_off), o, b->bpc, st, &side);
     }
     e = hipStreamEndCapture(st, &g->graph);
+    gn::side_streams_destroy(&side);
     if (!rc && e == hipSuccess) e = hipGraphInstantiate(&g->exec, g->graph, nullptr, nullptr, 0);
     if (rc || e != hipSuccess) {
         if (g->graph) (void)hipGraphDestroy(g->graph);

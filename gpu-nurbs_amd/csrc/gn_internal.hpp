@@ -254,8 +254,6 @@ struct SideStreams {
     hipEvent_t fork = nullptr, join[kSideStreams] = {};
 };
 int side_streams_create(SideStreams *ss);
-// Creates the device's shared side-stream set (call before a graph capture).
-int batch_prepare();
 void side_streams_destroy(SideStreams *ss);
 // Per group range one launch (batch.hip), or the persistent launches of batch_refill.hip where their
 // rule says so (path_rules.hpp); a seed launch before the latter, and for nearest-leaf seeds.  The

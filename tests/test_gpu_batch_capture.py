@@ -55,3 +55,50 @@ def test_replays_give_the_eager_bits(per, tile, seed):
         for a, e in zip(out, eager):
             assert torch.equal(a.view(torch.uint8), e.view(torch.uint8)), rep
     b.close()
+
+
+def test_graphs_are_made_beside_eager_calls():
+    """One thread captures batch graphs while another makes calls whose groups take the side streams: every
+    call and every replay gives its bits."""
+    import threading
+
+    surfs, b = _batch()
+    counts = [500 + 7 * k for k in range(len(surfs))]
+    n = sum(counts)
+    segs = G.segments(np.arange(len(surfs)), counts)
+    P = torch.rand(3, n, dtype=torch.float64, generator=torch.Generator().manual_seed(5)).cuda()
+    x, y, z = (t.contiguous() for t in P)
+    o = G.default_opts(seed_mode=G.SEED_GRID_STEP, **MIXED)
+    ref = [t.clone() for t in b.invert(segs, x, y, z, o)]
+    new = lambda: [torch.zeros(n, dtype=t.dtype, device="cuda") for t in ref]  # noqa: E731
+    eager, errors, stop = [new() for _ in range(300)], [], threading.Event()
+    torch.cuda.synchronize()
+
+    def calls():
+        st = torch.cuda.Stream()
+        try:
+            for out in eager:
+                b.invert(segs, x, y, z, o, out=out, stream=st)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+        st.synchronize()
+        stop.set()
+
+    st, outs, graphs = torch.cuda.Stream(), [], []
+    t = threading.Thread(target=calls)
+    t.start()
+    while not stop.is_set() or len(graphs) < 4:
+        outs.append(new())
+        st.wait_stream(torch.cuda.current_stream())
+        graphs.append(b.graph(segs, x, y, z, *outs[-1], o, stream=st))
+        graphs[-1].launch(stream=st)
+        if len(graphs) == 60:
+            break
+    t.join()
+    torch.cuda.synchronize()
+    assert not errors, errors
+    for k, out in enumerate(eager + outs):
+        assert all(torch.equal(a.view(torch.uint8), r.view(torch.uint8)) for a, r in zip(out, ref)), k
+    for g in graphs:
+        g.close()
+    b.close()

@@ -157,6 +157,20 @@ struct EvalLaunch {
     //     order 2, 4,194,305 107 / 138 / 183 / 227: one.
     // Rows a multiple of 64 MiB apart start on the same channels: four tiles lose to two, FP64 (3,3) order 2
     // 16,777,216 points 837 / 800, FP32 482 / 462.
+    // All that holds over many rounds.  Where one round of the resident blocks takes all the points, it has no
+    // last round that is part empty, and over (2,2) to (5,5) and orders 0 to 3, 131,072 to 1,500,001 points, it wins
+    // up to eight tiles, us for that against the number above: FP64 (3,3) order 2, 800,000 points 41.9 / 45.4, order 3
+    // 51.1 / 56.3, FP32 (2,5) order 2 27.4 / 31.8.  On rows of partial lines up to seven, and only where the rule
+    // above has four for FP32 ((5,5) order 1, 800,003 points 0.80 of the time; where it has two or one, 1.0 to 1.3)
+    // and two for FP64 ((4,4) order 3, 300,003 34 / 48; eight tiles 1.03 to 1.08); where it has one, two rounds only:
+    // FP64 (2,2) order 2, 200,003 14.5 / 16.8, three 1.15.  FP32 waves of two tiles leave the last round half empty
+    // where the rounds are odd: with one, (5,5) order 3, 300,003 24.8 / 27.4, (2,5) order 2, 800,003 28.2 / 30.0, (4,4)
+    // order 2, 400,001 23.6 / 24.7; at order 1 two stay ahead, (2,2) 800,003 0.95.
+    static bool one_round(size_t tiles, size_t most, size_t n) {
+        if (n % (128 / sizeof(T)) == 0) return most > 1 && tiles <= 8;
+        if (sizeof(T) == 4) return most == 4 && tiles <= 7;
+        return most > 1 ? tiles <= 7 : tiles == 2;
+    }
     static size_t most_tiles(int entries, int order, size_t n) {
         const size_t fields = order == 0 ? 3 : order == 1 ? 9 : order == 2 ? 18 : 30;
         const double per = (double)(fields * sizeof(T)) / entries;  // bytes written per patch entry
@@ -169,6 +183,9 @@ struct EvalLaunch {
         const bool four = per < (sizeof(T) == 8 ? 15.5 : 7.8), two = per < (sizeof(T) == 8 ? 20 : 10);
         return four && !(order >= 2 && n * sizeof(T) % ((size_t)1 << 26) == 0) ? 4 : two ? 2 : 1;
     }
+    static bool odd_rounds(size_t tiles, size_t most, size_t n) {
+        return sizeof(T) == 4 && n % 32 != 0 && most == 2 && tiles % 2 == 1 && tiles <= 7;
+    }
     template <int K1, int K2, int ORDER>
     int rows() {
         auto k = k_eval_rows<K1, K2, ORDER, T, TP>;
@@ -177,7 +194,8 @@ struct EvalLaunch {
         const size_t resident = blocks > cus ? cus * blocks_per_cu((const void *)k, kRowBlock) : cus;
         const size_t most = most_tiles(K1 * K2, ORDER, n);
         size_t tiles = (blocks + resident - 1) / resident;
-        tiles = tiles < most ? tiles : most;
+        if (ORDER >= 2 && odd_rounds(tiles, most, n)) tiles = 1;
+        if (!one_round(tiles, most, n)) tiles = tiles < most ? tiles : most;
         if (tiles < n >> 31) tiles = n >> 31;  // a grid holds below 2^32 lanes
         if (tiles < 1) tiles = 1;
         const unsigned grid = (unsigned)((blocks + tiles - 1) / tiles);

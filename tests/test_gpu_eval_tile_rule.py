@@ -57,3 +57,34 @@ def test_partial_lines():
 
     whole, part = best(12_000_032), best(12_000_007)
     assert part < 1.12 * whole, (part, whole)
+
+
+@pytest.mark.parametrize("p,q,order,dtype,n", [
+    (2, 5, 2, torch.float32, 800_000), (5, 5, 1, torch.float32, 800_003), (5, 5, 3, torch.float32, 300_003),
+    (4, 4, 3, torch.float64, 300_003), (4, 4, 3, torch.float64, 458_752 - 1),
+    (2, 2, 2, torch.float64, 200_003), (3, 3, 2, torch.float64, 1 << 20)])
+def test_bits_in_one_round(p, q, order, dtype, n):
+    test_bits_at_every_number_of_tiles(p, q, order, dtype, n)
+
+
+def test_one_round():
+    """FP64 patches of 25 entries run a block per CU.  Five tiles per wave take 300,003 points in one round,
+    5/4 of the time of the 262,139 that four take; with four there is a second round for the rest, which
+    waves of four tiles cannot share: 1.6 times and more."""
+    s = _surface(4, 4, 40)
+
+    def best(n):
+        u, v = torch.rand(2, n, dtype=torch.float64, device="cuda")
+        out = torch.empty((30, n), dtype=torch.float64, device="cuda")
+        t = []
+        for _ in range(7):
+            torch.cuda.synchronize()
+            t0 = time.perf_counter()
+            for _ in range(20):
+                s.Evaluate(u, v, 3, precision=G.GN_FP64, out=out)
+            torch.cuda.synchronize()
+            t.append(time.perf_counter() - t0)
+        return min(t[1:])
+
+    four, five = best(262_139), best(300_003)
+    assert five < 1.42 * four, (five, four)

@@ -195,7 +195,12 @@ struct EvalLaunch {
         const size_t most = most_tiles(K1 * K2, ORDER, n);
         size_t tiles = (blocks + resident - 1) / resident;
         if (ORDER >= 2 && odd_rounds(tiles, most, n)) tiles = 1;
-        if (!one_round(tiles, most, n)) tiles = tiles < most ? tiles : most;
+        // the rounds that `most` tiles would take, evenly filled: FP64 (4,4) order 0, 600,001 points are 10 tiles for
+        // each resident wave, two rounds of 5 45 us, 8 and a rest 65; order 0 (3,3) 1,500,000, 12, 52 and 55
+        if (tiles > most && !one_round(tiles, most, n)) {
+            const size_t rounds = (tiles + most - 1) / most;
+            tiles = (tiles + rounds - 1) / rounds;
+        }
         if (tiles < n >> 31) tiles = n >> 31;  // a grid holds below 2^32 lanes
         if (tiles < 1) tiles = 1;
         const unsigned grid = (unsigned)((blocks + tiles - 1) / tiles);

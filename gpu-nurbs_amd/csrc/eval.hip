@@ -154,7 +154,8 @@ struct EvalLaunch {
     //     order 2 168 / 235 / 245 / 248: one.  Patches of more than 20 entries, a block per CU: (5,4) order 3, 1,000,003
     //     120 / 107 / 98 / 94: eight; (4,4) order 3, 4,194,305 426 / 380 / 393 / 462, 8,388,613 998 / 802 / 786 / 745: four.
     //   FP32 (3,3) order 1, 5,000,003 108 / 98 / 93 / 94: four; (4,4) order 2, 2,000,005 78 / 74 / 77 / 85: two; (3,3)
-    //     order 2, 4,194,305 107 / 138 / 183 / 227: one.
+    //     order 2, 4,194,305 107 / 138 / 183 / 227: one.  (2,5) order 2 lies between, 2,000,005 points 61 / 66 / 70 / 77,
+    //     4,194,305 128 / 130, 8,388,613 248 / 226: two from 6 M points.
     // Rows a multiple of 64 MiB apart start on the same channels: four tiles lose to two, FP64 (3,3) order 2
     // 16,777,216 points 837 / 800, FP32 482 / 462.
     // All that holds over many rounds.  Where one round of the resident blocks takes all the points, it has no
@@ -164,8 +165,8 @@ struct EvalLaunch {
     // above has four for FP32 ((5,5) order 1, 800,003 points 0.80 of the time; where it has two or one, 1.0 to 1.3)
     // and two for FP64 ((4,4) order 3, 300,003 34 / 48; eight tiles 1.03 to 1.08); where it has one, two rounds only:
     // FP64 (2,2) order 2, 200,003 14.5 / 16.8, three 1.15.  FP32 waves of two tiles leave the last round half empty
-    // where the rounds are odd: with one, (5,5) order 3, 300,003 24.8 / 27.4, (2,5) order 2, 800,003 28.2 / 30.0, (4,4)
-    // order 2, 400,001 23.6 / 24.7; at order 1 two stay ahead, (2,2) 800,003 0.95.
+    // where the rounds are odd: with one, (5,5) order 3, 300,003 24.8 / 27.4, (4,4) order 2, 400,001 23.6 /
+    // 24.7; at order 1 two stay ahead, (2,2) 800,003 0.95.
     static bool one_round(size_t tiles, size_t most, size_t n) {
         if (n % (128 / sizeof(T)) == 0) return most > 1 && tiles <= 8;
         if (sizeof(T) == 4) return most == 4 && tiles <= 7;
@@ -175,7 +176,7 @@ struct EvalLaunch {
         const size_t fields = order == 0 ? 3 : order == 1 ? 9 : order == 2 ? 18 : 30;
         const double per = (double)(fields * sizeof(T)) / entries;  // bytes written per patch entry
         if (n % (128 / sizeof(T)) != 0) {
-            if (sizeof(T) == 4) return per < 2.5 ? 4 : per < 4.4 ? 2 : 1;
+            if (sizeof(T) == 4) return per < 2.5 ? 4 : per < (order >= 2 && n < 6000000 ? 3.7 : 4.4) ? 2 : 1;
             if (entries > 20) return per < 9 ? 8 : 4;
             return per < 7 ? 8 : per < 14 ? 2 : 1;
         }

@@ -63,7 +63,8 @@ def test_partial_lines():
     (2, 5, 2, torch.float32, 800_000), (5, 5, 1, torch.float32, 800_003), (5, 5, 3, torch.float32, 300_003),
     (4, 4, 3, torch.float64, 300_003), (4, 4, 3, torch.float64, 458_752 - 1),
     (2, 2, 2, torch.float64, 200_003), (3, 3, 2, torch.float64, 1 << 20), (4, 4, 0, torch.float64, 600_001),
-    (3, 3, 1, torch.float64, 1_500_001), (4, 4, 2, torch.float32, 1_500_007)])
+    (3, 3, 1, torch.float64, 1_500_001), (4, 4, 2, torch.float32, 1_500_007), (2, 5, 2, torch.float32, 2_000_005),
+    (2, 5, 2, torch.float32, 6_000_001)])
 def test_bits_in_one_round(p, q, order, dtype, n):
     test_bits_at_every_number_of_tiles(p, q, order, dtype, n)
 
